@@ -96,6 +96,10 @@ struct GemmArgs {
 };
 
 int launch_grouped_gemm(const GemmArgs& a, hipStream_t s);
+// fp32 GEMMs on the fp32 matrix instruction (smoe_gemm_f32.hip): K % 32 == 0,
+// rows and group strides of 16-byte multiples, aligned operands; no SwiGLU
+bool gemm_f32_fits(const GemmArgs& a);
+int launch_gemm_f32(const GemmArgs& a, hipStream_t s);
 // true when launch_grouped_gemm runs `a` on a ping-pong kernel, which reads
 // At and writes out_tiles (the fields themselves are ignored here)
 bool gemm_takes_row_tiles(const GemmArgs& a);

@@ -218,6 +218,28 @@ bool prefill_front_ok(const smoe_block* b, int N) {
          (b->H + b->L) % 8 == 0;
 }
 
+// Steps between decode and prefill size at E <= 16 (and fp32 steps of any
+// size up to it): the same outputs from two launches, the dense logits on
+// 16-row tiles (launch_front_dense) and one workgroup per chunk for the rest
+// (launch_route_chunk), then one launch for both plans.  The line is where
+// the separate stages would run a one-workgroup plan (C * E <= 512): they
+// took six launches, 52 us of a bf16 loop at 777 tokens and 61 us of an fp32
+// one at 2048 (E 8), against 25 and 21 us for the three; past it the
+// prefill front reads h once instead of once per 16 channels.
+// The logits wait in the proj region and the second plan's counts in act
+// (both written later in the loop), so the workspace is no larger.
+bool dense_front_ok(const smoe_block* b, int N) {
+  const int E = b->E, S = (E < b->K * b->M) ? E : b->K * b->M;
+  const int64_t C = (static_cast<int64_t>(N) + 63) / 64, n = N, ldf = E + E * E;
+  const bool f32 = b->act_dtype == SMOE_F32;
+  const int64_t fsz = ffn_dtype_of(b->experts) == SMOE_F32 ? 4 : 2;
+  auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  return N >= 1 && C * E <= 512 && C <= 64 && E % 4 == 0 && E <= 16 && b->K <= 16 && b->M <= 16 &&
+         2 * b->M <= E && b->H % (f32 ? 32 : 64) == 0 && (b->H + b->L) % (f32 ? 4 : 8) == 0 &&
+         a16(b->router_w) && a16(b->edge_gen_w) && ldf * 4 <= S * static_cast<int64_t>(b->H) * (f32 ? 4 : 2) &&
+         16 * C * E <= n * b->K * b->experts.U * fsz;
+}
+
 // Router logits (G == 0, f32 out): bf16 batches of >= 64 row tiles on the
 // one-pass logits kernel (a workgroup per 64 rows and every channel, h read
 // once: C3's 16384 x 1024 -> 32 logits 24 -> ~8 us), the rest on the
@@ -442,7 +464,10 @@ int block_forward(const smoe_block* b, const void* h_in, const void* x0, void* h
 
   const bool dec = decode_ok(b, N);
   const bool front = front_ok(b, N);
-  const bool pfront = !dec && !front && prefill_front_ok(b, N);
+  const bool dfront = !dec && !front && dense_front_ok(b, N) &&
+                      (reinterpret_cast<uintptr_t>(h_in) & 15) == 0 &&
+                      (reinterpret_cast<uintptr_t>(h_out) & 15) == 0;
+  const bool pfront = !dec && !front && !dfront && prefill_front_ok(b, N);
   const int32_t* active = gate ? gate->active : nullptr;
   const void* cur = h_in;
   for (int i = 0; i < num_loops; ++i) {
@@ -603,14 +628,15 @@ int block_forward(const smoe_block* b, const void* h_in, const void* x0, void* h
                                at<int32_t>(ws, l.d_rows), at<float>(ws, l.d_roww),
                                at<int32_t>(ws, l.d_tokrow), active, s),
             "front routing");
-    } else if (pfront) {
-      // 1-6 in one launch per 64-token chunk (logits of the router and every
-      // edge generator row, top-k, per-source top-m, destination
-      // coefficients, both plans' chunk ranks), then the plans' scan and
-      // scatter, which also moves the per-source edges (slot order, in the
-      // edge_logit region meanwhile) to their expert-plan rows
+    } else if (pfront || dfront) {
+      // 1-6 per 64-token chunk (logits of the router and every edge
+      // generator row, top-k, per-source top-m, destination coefficients,
+      // both plans' chunk ranks) in one launch, or the logits and the rest
+      // in one each (dense_front_ok); then the plans' scan and scatter,
+      // which also moves the per-source edges (slot order, in the edge_logit
+      // region meanwhile) to their expert-plan rows
       GemmArgs fg;
-      fg.fmt = SMOE_BF16;
+      fg.fmt = gfmt;
       fg.epi = EPI_F32_BIAS;
       fg.A = cur;
       fg.lda = H;
@@ -626,7 +652,8 @@ int block_forward(const smoe_block* b, const void* h_in, const void* x0, void* h
       fg.n_split = E;
       fg.bias2 = b->edge_loop_bias + static_cast<int64_t>(r) * E * E;
       const int C = (N + 63) / 64;
-      int32_t* ccnt = at<int32_t>(ws, l.scratch);  // expert plan [E, C] x 2, then destination
+      // expert plan [E, C] x 2, then destination plan
+      int32_t* ccnt = at<int32_t>(ws, dfront ? l.act : l.scratch);
       FrontPrefill fp;
       fp.N = N;
       fp.E = E;
@@ -650,7 +677,15 @@ int block_forward(const smoe_block* b, const void* h_in, const void* x0, void* h
       fp.d_ccnt = ccnt + 2 * static_cast<int64_t>(C) * E;
       fp.d_cacnt = ccnt + 3 * static_cast<int64_t>(C) * E;
       fp.active = active;
-      STAGE(SMOE_STAGE_FRONT_GEMM, launch_front_prefill(fg, fp, s), "prefill front");
+      if (dfront) {
+        fg.out = at<float>(ws, l.proj);
+        fg.ldo = fg.N_out;
+        STAGE(SMOE_STAGE_FRONT_GEMM, launch_front_dense(fg, s), "dense front logits");
+        STAGE(SMOE_STAGE_FRONT_ROUTE, launch_route_chunk(at<float>(ws, l.proj), fg.N_out, fp, s),
+              "dense front routing");
+      } else {
+        STAGE(SMOE_STAGE_FRONT_GEMM, launch_front_prefill(fg, fp, s), "prefill front");
+      }
       PlanSpec pe, pd;
       pe.tok_g = fp.tok_e;
       pe.tok_w = fp.tok_ew;

@@ -184,6 +184,53 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   }
 }
 
+// Routing and ranking of one 64-token chunk by WAVES waves, the logits row of
+// chunk token r at row_of(r) (router, then every source's edges): top-k and
+// top-m per token, the tokens' sources and destinations also in LDS (s_e /
+// s_ew [64, K], s_d / s_dc [64, S <= 16]), then the chunk's ranks for both
+// plans.  Every thread of the workgroup calls it.
+template <int KB, int WAVES, typename Row>
+__device__ __forceinline__ void route_chunk(const FrontPrefill& f, int chunk, Row row_of,
+                                            int32_t* s_e, float* s_ew, int32_t* s_d, float* s_dc) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int N = f.N, E = f.E, K = f.K, t0 = chunk * kFlRows;
+  // passes of 4 tokens per wave, a segment of 16 lanes per token
+  const int e = lane & 15, le = e < E ? e : E - 1;
+#pragma unroll 1
+  for (int ps = 0; ps < kFlRows / (4 * WAVES); ++ps) {
+    const int tl = (kFlRows / WAVES) * wave + 4 * ps + (lane >> 4);
+    const int t = t0 + tl;
+    const bool ok = t < N;
+    const float* row = row_of(tl);
+    const float v = row[le];
+    const bool live = !f.active || f.active[ok ? t : N - 1] != 0;
+    uint64_t m = topk_seg<16>(v, t, ok, live, E, K, f.top_idx, f.top_w, f.tok_e, f.tok_ew, s_e,
+                              s_ew, tl);
+    if (!live) m = 0;  // a token that has left: no sources (tok_e holds -1)
+    float ev[KB];
+    int rw[KB];
+    bool lv[KB];
+#pragma unroll
+    for (int j = 0; j < KB; ++j) {  // the selected sources, ascending
+      const int sj = m ? __builtin_ctzll(m) : 0;
+      lv[j] = ok && j < K && m != 0;
+      m &= m - 1;
+      rw[j] = t * K + j;
+      ev[j] = row[E + sj * E + le];
+    }
+    topm_seg<16, KB>(ev, rw, lv, t, ok, E, f.M, f.S, f.slot_idx, f.slot_w, f.tok_d, f.tok_dc, s_d,
+                     s_dc, tl);
+  }
+  __syncthreads();
+  // 3 the chunk's ranks: wave 0 the expert plan, wave 1 the destination plan
+  if (wave == 0)
+    rank_chunk(s_e, s_ew, N, K, E, 0, t0, 0, 64, f.e_ccnt + chunk, f.e_cacnt + chunk, f.C,
+               f.e_tokrow, t0);
+  else if (wave == 1)
+    rank_chunk(s_d, s_dc, N, f.S, E, 1, t0, 0, 64, f.d_ccnt + chunk, f.d_cacnt + chunk, f.C,
+               f.d_tokrow, t0);
+}
+
 // The one-pass prefill front (E <= 16): a workgroup's 64 tokens are one
 // chunk of the dispatch plans, so after its logits GEMM the workgroup also
 // routes them and ranks them for both plans, with the logits in LDS.  Eight
@@ -223,7 +270,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   float* s_ew = reinterpret_cast<float*>(s_e + kFlRows * KB);      // and weights
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int q = lane >> 4, l16 = lane & 15;
-  const int N = f.N, E = f.E, K = f.K, ldf = p.N_out;
+  const int N = f.N, E = f.E, ldf = p.N_out;
   const int chunk = blockIdx.x, t0 = chunk * kFlRows;
   const int NT = (p.N_out + 15) >> 4;
   f32x4 acc[TPW][4];
@@ -252,41 +299,29 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   }
   __syncthreads();
-  // 2 routing: 2 passes of 4 tokens per wave
-  const int e = lane & 15, le = e < E ? e : E - 1;
-#pragma unroll 1
-  for (int ps = 0; ps < kFlRows / (4 * kFpWaves); ++ps) {
-    const int tl = (kFlRows / kFpWaves) * wave + 4 * ps + (lane >> 4);
-    const int t = t0 + tl;
-    const bool ok = t < N;
-    const float* row = ft + tl * ldf;
-    const float v = row[le];
-    const bool live = !f.active || f.active[ok ? t : N - 1] != 0;
-    uint64_t m = topk_seg<16>(v, t, ok, live, E, K, f.top_idx, f.top_w, f.tok_e, f.tok_ew, s_e,
-                              s_ew, tl);
-    if (!live) m = 0;  // a token that has left: no sources (tok_e holds -1)
-    float ev[KB];
-    int rw[KB];
-    bool lv[KB];
-#pragma unroll
-    for (int j = 0; j < KB; ++j) {  // the selected sources, ascending
-      const int sj = m ? __builtin_ctzll(m) : 0;
-      lv[j] = ok && j < K && m != 0;
-      m &= m - 1;
-      rw[j] = t * K + j;
-      ev[j] = row[E + sj * E + le];
-    }
-    topm_seg<16, KB>(ev, rw, lv, t, ok, E, f.M, f.S, f.slot_idx, f.slot_w, f.tok_d, f.tok_dc, s_d,
-                     s_dc, tl);
-  }
-  __syncthreads();
-  // 3 the chunk's ranks: wave 0 the expert plan, wave 1 the destination plan
-  if (wave == 0)
-    rank_chunk(s_e, s_ew, N, K, E, 0, t0, 0, 64, f.e_ccnt + chunk, f.e_cacnt + chunk, f.C,
-               f.e_tokrow, t0);
-  else if (wave == 1)
-    rank_chunk(s_d, s_dc, N, f.S, E, 1, t0, 0, 64, f.d_ccnt + chunk, f.d_cacnt + chunk, f.C,
-               f.d_tokrow, t0);
+  // 2, 3
+  route_chunk<KB, kFpWaves>(f, chunk, [&](int tl) { return ft + tl * ldf; }, s_e, s_ew, s_d, s_dc);
+}
+
+// The dense front's second launch (16-row logits tiles instead of whole
+// chunks, launch_front_dense): steps 2 and 3 above on the [N, E + E*E]
+// logits in memory, one workgroup per chunk, 16 waves so that its 64 tokens
+// are routed in one pass.  Bound: latency (two dependent reads of the logits
+// rows, then one wave's ranking); it replaces the top-k, edge-logit, top-m
+// and first plan launches of the separate stages.
+template <int KB>
+__global__ __launch_bounds__(1024) void k_route_chunk(const float* __restrict__ front, int ldf,
+                                                      const FrontPrefill f) {
+  __shared__ int32_t s_d[kFlRows * 16], s_e[kFlRows * KB];
+  __shared__ float s_dc[kFlRows * 16], s_ew[kFlRows * KB];
+  const int t0 = blockIdx.x * kFlRows;
+  const int tl = threadIdx.x >> 4, e = threadIdx.x & 15;  // the token this segment routes
+  if (t0 + tl < f.N && e < f.E)
+    f.logits[static_cast<int64_t>(t0 + tl) * f.E + e] = front[static_cast<int64_t>(t0 + tl) * ldf + e];
+  route_chunk<KB, 16>(
+      f, blockIdx.x,
+      [&](int r) { return front + static_cast<int64_t>(min(t0 + r, f.N - 1)) * ldf; }, s_e, s_ew,
+      s_d, s_dc);
 }
 
 int launch_front_logits(const GemmArgs& a, hipStream_t s) {
@@ -344,6 +379,21 @@ int launch_front_prefill(const GemmArgs& a, const FrontPrefill& f, hipStream_t s
   }
 #undef SMOE_FP_K
 #undef SMOE_FP
+  return hipGetLastError() == hipSuccess ? SMOE_OK : SMOE_EHIP;
+}
+
+int launch_route_chunk(const float* front, int ldf, const FrontPrefill& f, hipStream_t s) {
+  if (f.E < 4 || f.E > 16 || f.E % 4 || ldf < f.E + f.E * f.E || f.N < 1 || f.K < 1 || f.K > f.E ||
+      f.M < 1 || f.M > f.E || f.S < 1 || f.S > f.E || f.C != (f.N + kFlRows - 1) / kFlRows)
+    return SMOE_EINVAL;
+  if (!front || !f.logits || !f.top_idx || !f.top_w || !f.tok_e || !f.tok_ew || !f.slot_idx ||
+      !f.slot_w || !f.tok_d || !f.tok_dc || !f.e_tokrow || !f.d_tokrow || !f.e_ccnt ||
+      !f.e_cacnt || !f.d_ccnt || !f.d_cacnt)
+    return SMOE_EINVAL;
+  const dim3 grid(static_cast<unsigned>(f.C)), block(1024);
+  if (f.K <= 2) SMOE_LAUNCH(k_route_chunk<2>, grid, block, 0, s, front, ldf, f);
+  else if (f.K <= 4) SMOE_LAUNCH(k_route_chunk<4>, grid, block, 0, s, front, ldf, f);
+  else SMOE_LAUNCH(k_route_chunk<16>, grid, block, 0, s, front, ldf, f);
   return hipGetLastError() == hipSuccess ? SMOE_OK : SMOE_EHIP;
 }
 

@@ -2444,6 +2444,17 @@ int launch_front_gemm(const GemmArgs& a, hipStream_t s) {
   return launch_skinny_fmt<SMOE_BF16, 1, 1, 4, 4>(a, s);
 }
 
+int launch_front_dense(const GemmArgs& a, hipStream_t s) {
+  if (a.epi != EPI_F32_BIAS || a.G != 0 || a.single_rows < 1 || !a.A || !a.W || !a.W2 || !a.out ||
+      a.N_out <= 0 || a.n_split < 0 || a.n_split > a.N_out || a.n_split % 4 || a.N_out % 4 || a.ldo % 4)
+    return SMOE_EINVAL;
+  if (a.fmt == SMOE_F32) return launch_gemm_f32_front(a, s);
+  if (a.fmt != SMOE_BF16 || a.K % 64 || a.lda % 8 || a.ldw % 8 || a.ldw2 % 8) return SMOE_EINVAL;
+  // the front GEMM's tiles: every output is summed as the separate stages'
+  // skinny GEMMs sum it, so the logits keep their bits
+  return launch_skinny_fmt<SMOE_BF16, 1, 1, 4, 4>(a, s);
+}
+
 // CUs of the current device (cached per device; 0 if unknown).
 int device_cus() {
   static int cus[64] = {0};

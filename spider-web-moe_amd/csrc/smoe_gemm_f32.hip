@@ -159,9 +159,13 @@ __global__ __launch_bounds__(256) void k_gemm_f32_skinny(const GemmArgs p) {
   const float* arow = reinterpret_cast<const float*>(p.A) + static_cast<int64_t>(ar) * p.lda + 4 * q;
   const float* wrow[TN];
 #pragma unroll
-  for (int t = 0; t < TN; ++t)
-    wrow[t] = reinterpret_cast<const float*>(p.W) + g * p.w_gstride +
-              static_cast<int64_t>(min(n0 + 16 * t + l16, p.N_out - 1)) * p.ldw + 4 * q;
+  for (int t = 0; t < TN; ++t) {
+    const int n = min(n0 + 16 * t + l16, p.N_out - 1);
+    wrow[t] = (p.W2 && n >= p.n_split)
+                  ? reinterpret_cast<const float*>(p.W2) + static_cast<int64_t>(n - p.n_split) * p.ldw2 + 4 * q
+                  : reinterpret_cast<const float*>(p.W) + g * p.w_gstride +
+                        static_cast<int64_t>(n) * p.ldw + 4 * q;
+  }
   f32x4 acc[TN];
 #pragma unroll
   for (int t = 0; t < TN; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -230,6 +234,18 @@ bool gemm_f32_fits(const GemmArgs& a) {
   const auto odd = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 != 0; };
   return a.fmt == SMOE_F32 && a.epi != EPI_SWIGLU && a.K % 32 == 0 && a.lda % 4 == 0 &&
          a.ldw % 4 == 0 && a.w_gstride % 4 == 0 && !odd(a.A) && !odd(a.W);
+}
+
+// The logits of [router | edge generator] rows (two weight segments): the
+// kernel the separate stages' logits (N_out = E <= 16) run on, which sums
+// every output in the same order whatever its strip.
+int launch_gemm_f32_front(const GemmArgs& a, hipStream_t s) {
+  if (!gemm_f32_fits(a) || a.ldw2 % 4 || reinterpret_cast<uintptr_t>(a.W2) % 16 ||
+      reinterpret_cast<uintptr_t>(a.out) % 16)
+    return SMOE_EINVAL;
+  SMOE_LAUNCH((k_gemm_f32_skinny<EPI_F32_BIAS, 1>),
+              dim3((a.single_rows + 15) / 16, (a.N_out + 15) / 16), dim3(256), 0, s, a);
+  return hipGetLastError() == hipSuccess ? SMOE_OK : SMOE_EHIP;
 }
 
 int launch_gemm_f32(const GemmArgs& a, hipStream_t s) {

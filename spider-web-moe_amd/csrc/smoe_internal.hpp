@@ -73,7 +73,7 @@ struct GemmArgs {
   const float* bias = nullptr;
   int64_t bias_gstride = 0;
   const float* row_scale = nullptr;
-  // optional second weight segment (launch_front_gemm only): output channels
+  // optional second weight segment (the front launches only): output channels
   // n >= n_split take row n - n_split of W2 (ldw2 elements apart) and bias2
   const void* W2 = nullptr;
   int ldw2 = 0;
@@ -100,6 +100,7 @@ int launch_grouped_gemm(const GemmArgs& a, hipStream_t s);
 // rows and group strides of 16-byte multiples, aligned operands; no SwiGLU
 bool gemm_f32_fits(const GemmArgs& a);
 int launch_gemm_f32(const GemmArgs& a, hipStream_t s);
+int launch_gemm_f32_front(const GemmArgs& a, hipStream_t s);  // W2: launch_front_dense
 // true when launch_grouped_gemm runs `a` on a ping-pong kernel, which reads
 // At and writes out_tiles (the fields themselves are ignored here)
 bool gemm_takes_row_tiles(const GemmArgs& a);
@@ -154,7 +155,8 @@ struct PlanSpec {
   int pay_m = 0;
 };
 // The scan and scatter of two plans over the same N tokens whose chunk
-// counts and ranks are in place (launch_front_prefill): one launch each.
+// counts and ranks are in place (launch_front_prefill, launch_route_chunk):
+// one launch each, or one for both (few chunks).
 // scratch: plan a's [G, C] count and positive-count matrices, then plan
 // b's (plan_scratch_bytes(N, a.G) + plan_scratch_bytes(N, b.G)).
 int launch_plan2_finish(const PlanSpec& a, const PlanSpec& b, int N, void* scratch, hipStream_t s);
@@ -180,6 +182,11 @@ struct FrontPrefill {
 // = E, bias / bias2, N_out = E + E*E), then in the same workgroups top-k,
 // per-source top-m, destination coefficients and both plans' chunk ranks.
 int launch_front_prefill(const GemmArgs& a, const FrontPrefill& f, hipStream_t s);
+// The same in two launches for the steps between decode and prefill size,
+// bf16 and fp32: the dense logits [N, ldo] on 16-row tiles (a as above, with
+// out), then top-k, top-m and both plans' chunk ranks from them.
+int launch_front_dense(const GemmArgs& a, hipStream_t s);
+int launch_route_chunk(const float* front, int ldf, const FrontPrefill& f, hipStream_t s);
 int launch_plan(const int32_t* tok_g, const float* tok_w, int N, int S, int G, int drop_nonpos,
                 int32_t* cnt, int32_t* acnt, int32_t* off, int32_t* rows, float* roww,
                 int32_t* tokrow, void* scratch, hipStream_t s);

@@ -859,6 +859,29 @@ struct Plan2 {
   int pay_m;
 };
 
+// Workgroup blk of a plan's scatter: its 256 tokens' rows from the group
+// offsets, the chunk prefixes base [G, C] and the ranks in tokrow; the first
+// workgroup also writes the offsets.
+template <typename P>
+__device__ __forceinline__ void scatter_block(const Plan2& p, int blk, int N, P base, int C,
+                                              const int* goff) {
+  if (blk == 0)
+    for (int g = threadIdx.x; g <= p.G; g += 256) p.off[g] = goff[g];
+  const int t = blk * 256 + threadIdx.x;
+  if (t >= N) return;
+  scatter_token(p.tok_g, p.tok_w, t, p.S, p.G, base + (t >> 6), C, goff, p.rows, p.roww, p.tokrow);
+  if (p.pay_m <= 0) return;
+  const int64_t e0 = static_cast<int64_t>(t) * p.S;
+  for (int j = 0; j < p.S; ++j) {
+    const int row = p.tokrow[e0 + j];  // this thread's own store above: -1 for dropped entries
+    if (row < 0) continue;
+    for (int i = 0; i < p.pay_m; ++i) {
+      p.out_idx[static_cast<int64_t>(row) * p.pay_m + i] = p.pay_idx[(e0 + j) * p.pay_m + i];
+      p.out_w[static_cast<int64_t>(row) * p.pay_m + i] = p.pay_w[(e0 + j) * p.pay_m + i];
+    }
+  }
+}
+
 __global__ __launch_bounds__(64) void k_plan2_scan(const Plan2 a, const Plan2 b, int C) {
   const bool second = static_cast<int>(blockIdx.x) >= a.G;
   const Plan2& p = second ? b : a;
@@ -872,21 +895,53 @@ __global__ __launch_bounds__(256) void k_plan2_scatter(const Plan2 a, const Plan
   const Plan2& p = second ? b : a;
   const int blk = second ? blockIdx.x - nb : blockIdx.x;
   block_group_offsets(p.cnt, p.G, goff, wsum);
-  if (blk == 0)
-    for (int g = threadIdx.x; g <= p.G; g += 256) p.off[g] = goff[g];
-  const int t = blk * 256 + threadIdx.x;
-  if (t >= N) return;
-  scatter_token(p.tok_g, p.tok_w, t, p.S, p.G, p.ccnt + (t >> 6), C, goff, p.rows, p.roww, p.tokrow);
-  if (p.pay_m <= 0) return;
-  const int64_t e0 = static_cast<int64_t>(t) * p.S;
-  for (int j = 0; j < p.S; ++j) {
-    const int row = p.tokrow[e0 + j];  // this thread's own store above: -1 for dropped entries
-    if (row < 0) continue;
-    for (int i = 0; i < p.pay_m; ++i) {
-      p.out_idx[static_cast<int64_t>(row) * p.pay_m + i] = p.pay_idx[(e0 + j) * p.pay_m + i];
-      p.out_w[static_cast<int64_t>(row) * p.pay_m + i] = p.pay_w[(e0 + j) * p.pay_m + i];
+  scatter_block(p, blk, N, p.ccnt, C, goff);
+}
+
+// Both steps in one launch while a plan has at most 64 chunks over at most 16
+// groups: every workgroup scans the [G, C] counts itself (one lane per chunk,
+// a wave's four groups loaded together, 4 KB at most) instead of waiting for
+// a launch of G one-wave workgroups.  Past that the scan is launched once:
+// at 256 chunks, repeating it in every scatter workgroup cost more than the
+// launch (0.090 -> 0.116 ms over six loops).
+constexpr int kFinishMaxC = 64, kFinishMaxG = 16;
+
+__global__ __launch_bounds__(256) void k_plan2_finish(const Plan2 a, const Plan2 b, int N, int C) {
+  __shared__ int base[kFinishMaxG * kFinishMaxC], tot[kFinishMaxG];
+  __shared__ int goff[kFinishMaxG + 1], wsum[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int nb = (N + 255) / 256;
+  const bool second = static_cast<int>(blockIdx.x) >= nb;
+  const Plan2& p = second ? b : a;
+  const int blk = second ? blockIdx.x - nb : blockIdx.x;
+  int v[kFinishMaxG / 4], av[kFinishMaxG / 4];
+#pragma unroll
+  for (int i = 0; i < kFinishMaxG / 4; ++i) {  // unconditional loads at clamped indices
+    const int g = wave + 4 * i, c = min(g, p.G - 1) * C + min(lane, C - 1);
+    const bool in = g < p.G && lane < C;
+    v[i] = p.ccnt[c];
+    av[i] = p.cacnt[c];
+    v[i] = in ? v[i] : 0;
+    av[i] = in ? av[i] : 0;
+  }
+#pragma unroll
+  for (int i = 0; i < kFinishMaxG / 4; ++i) {
+    const int g = wave + 4 * i;  // uniform
+    const int incl = wave_incl_scan(v[i]);
+    const int pos = __builtin_amdgcn_readlane(wave_incl_scan(av[i]), 63);
+    if (g >= p.G) continue;
+    if (lane < C) base[g * C + lane] = incl - v[i];
+    if (lane == 63) {
+      tot[g] = incl;
+      if (blk == 0) {
+        p.cnt[g] = incl;
+        p.acnt[g] = pos;
+      }
     }
   }
+  __syncthreads();
+  block_group_offsets(tot, p.G, goff, wsum);
+  scatter_block(p, blk, N, base, C, goff);
 }
 
 int launch_plan2_finish(const PlanSpec& pa, const PlanSpec& pb, int N, void* scratch,
@@ -922,8 +977,13 @@ int launch_plan2_finish(const PlanSpec& pa, const PlanSpec& pb, int N, void* scr
     q.out_w = p.out_w;
     q.pay_m = p.pay_m;
   }
-  hipLaunchKernelGGL(k_plan2_scan, dim3(a.G + b.G), dim3(64), 0, s, a, b, C);
-  hipLaunchKernelGGL(k_plan2_scatter, dim3(2 * ((N + 255) / 256)), dim3(256), 0, s, a, b, N, C);
+  const dim3 grid(2 * ((N + 255) / 256));
+  if (C <= kFinishMaxC && a.G <= kFinishMaxG && b.G <= kFinishMaxG) {
+    hipLaunchKernelGGL(k_plan2_finish, grid, dim3(256), 0, s, a, b, N, C);
+  } else {
+    hipLaunchKernelGGL(k_plan2_scan, dim3(a.G + b.G), dim3(64), 0, s, a, b, C);
+    hipLaunchKernelGGL(k_plan2_scatter, grid, dim3(256), 0, s, a, b, N, C);
+  }
   return hipGetLastError() == hipSuccess ? SMOE_OK : SMOE_EHIP;
 }
 

@@ -273,6 +273,39 @@ def test_block_small_steps_fused_front(n, e, k, m):
     assert int(rt["d_cnt"].sum()) == int((rt["tok_d"] >= 0).sum())
 
 
+@pytest.mark.parametrize("dtype,n,e,k,m", [("bf16", 65, 16, 2, 2), ("bf16", 128, 4, 1, 2),
+                                           ("bf16", 1000, 12, 3, 3), ("bf16", 2048, 16, 2, 2),
+                                           ("bf16", 600, 16, 5, 8), ("f32", 1, 8, 2, 3),
+                                           ("f32", 64, 8, 2, 3), ("f32", 65, 4, 2, 2),
+                                           ("f32", 2047, 16, 2, 4), ("f32", 4096, 8, 2, 3)])
+def test_block_dense_front(dtype, n, e, k, m):
+    """Steps between decode and prefill size at E <= 16 (C * E <= 512, C =
+    ceil(n / 64) chunks; fp32 from one token on): dense logits on 16-row
+    tiles, one workgroup per chunk for the routing and ranks, one launch for
+    both plans.  Sizes at the ends of the range, whole and partial chunks, k
+    above 4; against the oracle for two loops."""
+    from spider_moe_amd import _native as nat
+    from spider_moe_amd.workloads import make_block
+    say("dense front", dtype, n, e, k, m)
+    f32 = dtype == "f32"
+    # (at hidden 128 the logits of 16 experts would not fit the projection region)
+    wl = make_block("c1", tokens=n, hidden_size=256, num_experts=e, top_k=k, edges_per_expert=m,
+                    expert_ffn_size=256, num_loops=2, expert_activation="gelu" if f32 else "swiglu",
+                    experts=dtype, dtype=dtype)
+    timer = nat.StageTimer(stages=["router_gemm", "edge_logits", "front_gemm", "front_route"],
+                           capacity=64)
+    timer.start()
+    with torch.no_grad():
+        wl.layer(wl.h, wl.x0, 0)
+    assert set(timer.stop()) == {"front_gemm", "front_route"}
+    h = wl.h
+    for r in range(2):
+        h, rep = _check_loop(wl.layer, h, wl.x0, r, 1e-4 if f32 else 1e-2)
+    rt = wl.layer.last_routing()
+    assert int(rt["e_cnt"].sum()) == n * k
+    assert int(rt["d_cnt"].sum()) == int((rt["tok_d"] >= 0).sum())
+
+
 @pytest.mark.parametrize("n,e,k,m", [(2112, 16, 2, 2), (4160, 8, 2, 4), (8256, 4, 1, 2),
                                      (2800, 12, 3, 3), (4160, 32, 2, 2), (4096, 64, 2, 4)])
 def test_block_prefill_one_pass_logits(n, e, k, m):

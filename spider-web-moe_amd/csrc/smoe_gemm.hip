@@ -180,259 +180,6 @@ __global__ __launch_bounds__(WM* WN * 64) void k_gemm_mfma(const GemmArgs p) {
   }
 }
 
-// ------------------------------------------------ tile order, 4-wide out ----
-// Tile order of the large-tile kernels: the tile grid (real count, from the
-// plan) is split into 8 contiguous ranges, one per XCD (workgroup ids are
-// dealt to XCDs round robin), and each range is walked in super-rows of GM
-// m-tiles x all n-tiles so the super-row's A tiles stay in that XCD's L2
-// while weight tiles stream.
-template <int BM>
-__device__ __forceinline__ int count_m_tiles(const GemmArgs& p) {
-  return count_tiles(p, BM);
-}
-
-// Row tiles on 16-row bands (an operand or the output in the row-tile
-// layout): group g's tiles start at its first row rounded down to a multiple
-// of 16, BM rows apart; a tile's live rows are the group's, [rlo, rhi) in
-// tile rows.  A band shared by two groups is computed by a tile of each, and
-// each stores only its own rows.
-__device__ __forceinline__ void band_chunk(const GemmArgs& p, int BM, int b, int& lo, int& hi,
-                                           int& t) {
-  const int i = b + static_cast<int>(threadIdx.x & 63);
-  const int ic = i < p.G ? i : p.G - 1;
-  lo = p.grp_off[ic];
-  hi = p.grp_off[ic + 1];
-  t = (i < p.G && hi > lo) ? (hi - (lo & ~15) + BM - 1) / BM : 0;
-}
-
-__device__ __forceinline__ int count_band_tiles(const GemmArgs& p, int BM) {
-  if (p.G == 0) return (p.single_rows + BM - 1) / BM;
-  int total = 0;
-  for (int b = 0; b < p.G; b += 64) {
-    int lo, hi, t;
-    band_chunk(p, BM, b, lo, hi, t);
-    total += __builtin_amdgcn_readlane(wave_incl_scan(t), 63);
-  }
-  return total;
-}
-
-__device__ __forceinline__ bool find_band_tile(const GemmArgs& p, int BM, int tile, int& g, int& m0,
-                                               int& rlo, int& rhi) {
-  if (p.G == 0) {
-    int mrows;
-    if (!find_tile(p, BM, tile, g, m0, mrows)) return false;
-    rlo = 0;
-    rhi = mrows;
-    return true;
-  }
-  int acc = 0;
-  for (int b = 0; b < p.G; b += 64) {
-    int lo, hi, t;
-    band_chunk(p, BM, b, lo, hi, t);
-    const int incl = wave_incl_scan(t) + acc;
-    const uint64_t m = __ballot(tile < incl);
-    if (m) {
-      const int f = __builtin_ctzll(m);
-      g = b + f;
-      const int excl = __builtin_amdgcn_readlane(incl - t, f);
-      const int glo = __builtin_amdgcn_readlane(lo, f), ghi = __builtin_amdgcn_readlane(hi, f);
-      m0 = (glo & ~15) + (tile - excl) * BM;
-      rlo = max(glo - m0, 0);
-      rhi = min(ghi - m0, BM);
-      return true;
-    }
-    acc = __builtin_amdgcn_readlane(incl, 63);
-  }
-  return false;
-}
-
-__device__ __forceinline__ bool row_tiles(const GemmArgs& p) { return p.At != nullptr || p.out_tiles; }
-
-// The tile of workgroup bid: group, first row m0, live rows
-// [rlo, rhi) in tile rows (rlo > 0 only for band-aligned tiles), first
-// output channel.  Workgroup ids are dealt to the 8 XCDs round robin
-// (bid & 7 is the XCD).
-template <int BM, int BN, int GM>
-__device__ __forceinline__ bool big_tile(const GemmArgs& p, int bid, int& g, int& m0, int& rlo,
-                                         int& rhi, int& n0) {
-  const bool bands = row_tiles(p);
-  const int tn_count = (p.N_out + BN - 1) / BN;
-  const int tm_count = bands ? count_band_tiles(p, BM) : count_m_tiles<BM>(p);
-  const int T = tm_count * tn_count;
-  if (bid >= T) return false;
-  const int x = bid & 7, local = bid >> 3;
-  const int base = T >> 3, rem = T & 7;
-  const int logical = x * base + min(x, rem) + local;
-  const int grp = logical / (GM * tn_count);
-  const int first_m = grp * GM;
-  const int gsize = min(GM, tm_count - first_m);
-  const int in = logical - grp * GM * tn_count;
-  const int tm = first_m + in % gsize;
-  n0 = (in / gsize) * BN;
-  if (bands) return find_band_tile(p, BM, tm, g, m0, rlo, rhi);
-  int mrows;
-  if (!find_tile(p, BM, tm, g, m0, mrows)) return false;
-  rlo = 0;
-  rhi = mrows;
-  return true;
-}
-
-// Epilogue of an LDS-staged tile: math in registers, the bf16 tile staged
-// in the (idle) LDS ring, then coalesced 16-byte stores.  Staging layout:
-// row r, 16-byte chunk c at chunk c ^ (r & 15) (rows of OW bf16, no padding;
-// r & 7 for 8-chunk rows).  Only the live rows [rlo, rhi) are stored, and
-// 16-row strips without any are skipped.  With p.out_tiles the stores follow
-// the row-tile layout (m0 a multiple of 16): 64 consecutive threads write
-// one 1 KB block (16 rows x 32 columns).
-//
-// The lane's bias values (4 channels of each fragment column; SwiGLU: of its
-// up columns) and the row scales of its strips are loaded before any math
-// (one memory round trip for the whole epilogue).  The costly activations
-// (SwiGLU; GELU of small wave tiles) are computed into packed registers
-// before the workgroup barrier that frees the ring (the caller need not
-// synchronise), so one wave row's math overlaps the other's last MFMAs; the
-// others are computed as they are staged (a packed tile of 4 channels per
-// fragment column would not fit beside the accumulators).
-// Without a bias (the SwiGLU experts) its loads and adds are compiled out.
-// fp8 weights (WF): each channel's scale multiplies its accumulator first.
-template <int BM, int BN, int TM, int TN, int NT, int EPI, int WF = SMOE_BF16>
-__device__ __forceinline__ void tile_epilogue(const GemmArgs& p, const f32x4 (&acc)[TN / 16][TM / 16],
-                                              int g, int m0, int rlo, int rhi, int n0, int wm,
-                                              int wn, uint8_t* ring) {
-  constexpr int FM = TM / 16, FN = TN / 16;
-  constexpr int OW = (EPI == EPI_SWIGLU) ? BN / 2 : BN;  // output columns of the tile
-  constexpr int SWM = (OW / 8 >= 16 ? 16 : OW / 8) - 1;  // chunk swizzle mask
-  constexpr bool HAS_BIAS = EPI != EPI_ROWSCALE;
-  constexpr bool HAS_RS = EPI == EPI_ROWSCALE || EPI == EPI_DOWN;
-  constexpr int NJ = (EPI == EPI_SWIGLU) ? FN / 2 : FN;  // output fragment columns
-  constexpr bool EARLY = EPI == EPI_SWIGLU || (EPI == EPI_GELU && FM * NJ <= 16);
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int fr = lane & 15, fc = lane >> 4;
-  uint16_t* stg = reinterpret_cast<uint16_t*>(ring);
-  auto stg_at = [&](int r, int col) {  // staging row r, col: multiple of 4
-    return stg + r * OW + ((((col >> 3) ^ (r & SWM)) << 3) | (col & 7));
-  };
-  const int ncol0 = (EPI == EPI_SWIGLU) ? (n0 >> 1) : n0;
-  const int ncols = (EPI == EPI_SWIGLU) ? (p.N_out >> 1) : p.N_out;  // a last tile may be partial
-  auto live = [&](int i) {  // strip i holds a live row (wave-uniform)
-    const int tr0 = wm * TM + i * 16;
-    return tr0 < rhi && tr0 + 16 > rlo;
-  };
-  constexpr bool F8 = WF == SMOE_FP8_E4M3;
-  auto body = [&](auto with_bias) {
-    constexpr bool WB = HAS_BIAS && decltype(with_bias)::value;
-    float bq[WB ? NJ : 1][4];
-    float rsv[HAS_RS ? FM : 1];
-    // fp8 channel scales: [fragment column][channel] (SwiGLU: gate, then up 32 on)
-    float sc[F8 ? FN : 1][4];
-    if constexpr (F8) {
-#pragma unroll
-      for (int j = 0; j < FN; ++j) {
-        const int c = n0 + wn * TN + j * 16 + fc * 4;
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          sc[j][q] = c + q < p.N_out
-                         ? reinterpret_cast<const float*>(p.S)[g * p.s_gstride + c + q]
-                         : 0.f;
-      }
-    }
-    if constexpr (WB) {
-#pragma unroll
-      for (int j = 0, b = 0; j < FN; ++j) {
-        if (EPI == EPI_SWIGLU && (j & 3) >= 2) continue;
-        const int cl = wn * TN + j * 16 + fc * 4;
-        const int c = (EPI == EPI_SWIGLU) ? (n0 >> 1) + (cl >> 6) * 32 + (cl & 31) : n0 + cl;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) bq[b][q] = c + q < ncols ? bias_at(p, g, c + q) : 0.f;
-        ++b;
-      }
-    }
-    if constexpr (HAS_RS) {
-#pragma unroll
-      for (int i = 0; i < FM; ++i) {
-        const int lr = wm * TM + i * 16 + fr;
-        rsv[i] = lr >= rlo && lr < rhi ? p.row_scale[m0 + lr] : 0.f;
-      }
-    }
-    // the packed outputs of strip i, fragment column j (bias slot b)
-    auto value = [&](int i, int j, int b) {
-      float r[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        if constexpr (EPI == EPI_SWIGLU) {
-          const float gate = F8 ? acc[j][i][q] * sc[F8 ? j : 0][q] : acc[j][i][q];
-          const float up = F8 ? acc[j + 2][i][q] * sc[F8 ? j + 2 : 0][q] : acc[j + 2][i][q];
-          r[q] = silu(gate) * (WB ? up + bq[WB ? b : 0][q] : up);
-        } else {
-          const float v = F8 ? acc[j][i][q] * sc[F8 ? j : 0][q] : acc[j][i][q];
-          const float a = WB ? v + bq[WB ? b : 0][q] : v;
-          if constexpr (HAS_RS) r[q] = a * rsv[HAS_RS ? i : 0];
-          else if constexpr (EPI == EPI_GELU) r[q] = gelu_erf(a);
-          else r[q] = a;
-        }
-      }
-      return u32x2{pack_bf2(r[0], r[1]), pack_bf2(r[2], r[3])};
-    };
-    u32x2 pk[EARLY ? FM : 1][NJ];
-    if constexpr (EARLY) {
-#pragma unroll
-      for (int i = 0; i < FM; ++i) {
-        if (!live(i)) continue;
-#pragma unroll
-        for (int j = 0, b = 0; j < FN; ++j) {
-          if (EPI == EPI_SWIGLU && (j & 3) >= 2) continue;
-          pk[i][b] = value(i, j, b);
-          ++b;
-        }
-      }
-    }
-    __syncthreads();  // every wave is done with the ring: it becomes the staging buffer
-#pragma unroll
-    for (int i = 0; i < FM; ++i) {
-      if (!live(i)) continue;
-      const int sr = wm * TM + i * 16 + fr;  // staging row = tile row
-#pragma unroll
-      for (int j = 0, b = 0; j < FN; ++j) {
-        if (EPI == EPI_SWIGLU && (j & 3) >= 2) continue;
-        const int cl = wn * TN + j * 16 + fc * 4;  // channel within the tile
-        const int col = (EPI == EPI_SWIGLU) ? (cl >> 6) * 32 + (cl & 31) : cl;
-        *reinterpret_cast<u32x2*>(stg_at(sr, col)) = EARLY ? pk[EARLY ? i : 0][b] : value(i, j, b);
-        ++b;
-      }
-    }
-  };
-  if (!HAS_BIAS || p.bias) body(std::true_type{});
-  else body(std::false_type{});
-  __syncthreads();
-  uint16_t* out = reinterpret_cast<uint16_t*>(p.out);
-  if (p.out_tiles) {
-    constexpr int KB = OW / 32;  // 32-column blocks per tile row band
-    const int ldb = p.ldo >> 5;  // blocks per band of the whole output
-    for (int q = tid; q < BM / 16 * KB * 64; q += NT) {
-      const int blk = q >> 6, l = q & 63;
-      const int r = (blk / KB) * 16 + (l & 15), cc = (blk % KB) * 32 + (l >> 4) * 8;
-      if (r >= rlo && r < rhi && ncol0 + cc < ncols)
-        __builtin_nontemporal_store(
-            *reinterpret_cast<const u32x4*>(stg_at(r, cc)),
-            reinterpret_cast<u32x4*>(out + ((static_cast<int64_t>((m0 + r) >> 4) * ldb +
-                                             ((ncol0 + cc) >> 5)) << 9) + 8 * l));
-    }
-    return;
-  }
-  constexpr int CPR_OUT = OW / 8;  // 16-byte chunks per output row
-  for (int q = tid; q < BM * CPR_OUT; q += NT) {
-    const int r = q / CPR_OUT, cc = (q % CPR_OUT) * 8;
-    // non-temporal: every CU stores its tile at about the same time, and
-    // the burst streams past the caches (the next kernel reads it once).
-    // With the epilogue loads hoisted: C1's up GEMM 2.20 -> 2.15 ms per
-    // step, C3's step 3.66 -> 3.49 ms.
-    if (r >= rlo && r < rhi && ncol0 + cc < ncols)
-      __builtin_nontemporal_store(
-          *reinterpret_cast<const u32x4*>(stg_at(r, cc)),
-          reinterpret_cast<u32x4*>(out + static_cast<int64_t>(m0 + r) * p.ldo + ncol0 + cc));
-  }
-}
-
 // ------------------------------------------------- MFMA, LDS-DMA ring ----
 // 256 x BN block tile (BN = 256 or 128), 4 waves in a 2 x 2 grid, wave tile
 // 128 x BN/2.  K advances 32 per stage; operands go global -> LDS directly
@@ -888,13 +635,6 @@ __global__ __launch_bounds__(512, BM == 128 ? 2 : 1) void k_gemm_pp(const GemmAr
 // of all groups form one flat list (grid.y), so at many rows (router / edge
 // logits at prefill: narrow outputs, the activations are the stream) and
 // skewed groups the work still spreads evenly.
-// A lane's raw 16 consecutive k of one weight row, in its storage format
-// (only what the format needs stays in registers).
-template <int FMT> struct WRaw;
-template <> struct WRaw<SMOE_BF16> { u32x4 a, b; };
-template <> struct WRaw<SMOE_FP8_E4M3> { u32x4 a; };
-template <> struct WRaw<SMOE_INT4> { u32x2 a; float s; };  // 16 nibbles + their group scale
-
 template <int FMT>
 __device__ __forceinline__ WRaw<FMT> skinny_wload(const GemmArgs& p, const uint8_t* wrow, int k,
                                                   int g, int n) {
@@ -913,26 +653,6 @@ __device__ __forceinline__ WRaw<FMT> skinny_wload(const GemmArgs& p, const uint8
                      p.s_f16);
   }
   return r;
-}
-
-// The raw 16 k of a lane -> the bf16 A operands of the step's two MFMAs.
-template <int FMT>
-__device__ __forceinline__ void skinny_wconv(const WRaw<FMT>& r, bf16x8& lo, bf16x8& hi) {
-  u32x4 l, h;
-  if constexpr (FMT == SMOE_BF16) {
-    l = r.a;
-    h = r.b;
-  } else if constexpr (FMT == SMOE_FP8_E4M3) {
-    const u32x2 a0 = fp8x4_to_bf16x4(r.a.x), a1 = fp8x4_to_bf16x4(r.a.y);
-    const u32x2 b0 = fp8x4_to_bf16x4(r.a.z), b1 = fp8x4_to_bf16x4(r.a.w);
-    l = u32x4{a0.x, a0.y, a1.x, a1.y};
-    h = u32x4{b0.x, b0.y, b1.x, b1.y};
-  } else {
-    l = int4x8_to_bf16x8(r.a.x, r.s);
-    h = int4x8_to_bf16x8(r.a.y, r.s);
-  }
-  lo = __builtin_bit_cast(bf16x8, l);
-  hi = __builtin_bit_cast(bf16x8, h);
 }
 
 template <int FMT, int EPI, int TN, int RT, int NW, int U>
@@ -1497,220 +1217,44 @@ __global__ __launch_bounds__(256) void k_decode_edge(const GemmArgs p, const Dec
       p, blockIdx.y - 1, reinterpret_cast<f32x4*>(lds));
 }
 
-// ------------------------------------------------------- weight stream ----
-// Medium rows per group (a few dozen to ~128: mixed decode + prefill steps),
-// bf16 and fp8 weights (int4: k_gemm_stream4 below, the same work split).
-// The weights dominate the traffic and every weight is
-// used by all rows of its group, so a workgroup owns one group, a strip of
-// 256 output channels (wave w: channels 64 w .. 64 w + 63, four 16-channel
-// MFMA tiles) and the group's rows in passes of RT*16.  Both operands stream
-// global -> LDS by DMA (global_load_lds_dwordx4) through an NS-stage ring of
-// 64-wide K chunks, so the main loop's only vector-memory operations are the
-// DMAs and the explicit vmcnt waits stay exact:
-//   weights:     256 channel rows x 64 k in storage format (fp8 64 B, bf16
-//                128 B per row); a lane reads the 16 k at 16*(lane/16) of
-//                its channel and widens them to bf16
-//   activations: RT*16 rows x 64 k bf16 (128 B rows)
-//   MFMAs:       the step's two MFMAs take the low and the high 8 of the 16 k
-//                (the same permutation for both operands).
+// -------------------------------------------------- int4 weight stream ----
+// int4 weights at medium rows per group (a few dozen to ~128: mixed decode +
+// prefill steps).  The weights dominate the traffic and every weight is used
+// by all rows of its group, so a workgroup owns one group, a strip of 64 TN
+// output channels (a wave TN 16-channel MFMA tiles) and the group's rows in
+// passes of RT*16.  Both operands stream global -> LDS by DMA
+// (global_load_lds_dwordx4) through an NS-stage ring of 64-wide K chunks, so
+// the main loop's only vector-memory operations are the DMAs and the explicit
+// vmcnt waits stay exact; a chunk's two MFMAs take the low and the high 8 of
+// a lane's 16 k (the same permutation for both operands).
 // Every LDS row's 16-byte chunk c is stored at c ^ ((r / R) % C), C chunks
 // per row, R rows per 256 bytes: the 16 rows a ds_read phase touches then
 // cover all 64 banks once.  One barrier per chunk; chunk k+NS-1 is in flight
 // while chunk k computes.  Results go from registers to memory, 4
 // consecutive channels per lane.
-template <int FMT>
-constexpr int stream_wb() {  // bytes of one channel's 64-k slice
-  return FMT == SMOE_BF16 ? 128 : (FMT == SMOE_FP8_E4M3 ? 64 : 32);
-}
-constexpr int kStreamScaleMax = 4096;  // int4 scale-table entries per strip
-
-template <int FMT, int EPI, int RT, int NS, int WGS>
-__global__ __launch_bounds__(256, WGS) void k_gemm_stream(const GemmArgs p) {
-  constexpr int TN = 4;
-  constexpr int WB = stream_wb<FMT>();
-  constexpr int CPR = WB / 16;  // 16-byte chunks per weight row
-  constexpr int ROWS = RT * 16;
-  constexpr int W_BYTES = 256 * WB, A_BYTES = ROWS * 128, STAGE = W_BYTES + A_BYTES;
-  constexpr int W_LD = W_BYTES / 4096, A_LD = A_BYTES / 4096;  // DMA instructions per wave per stage
-  constexpr int LD = W_LD + A_LD;
-  constexpr int ESZ2 = FMT == SMOE_BF16 ? 4 : (FMT == SMOE_FP8_E4M3 ? 2 : 1);  // 2 x bytes/elt
-  static_assert(W_BYTES % 4096 == 0 && A_BYTES % 4096 == 0, "whole DMA instructions per wave");
-  static_assert(NS >= 3, "ring depth");
-  static_assert(EPI != EPI_SWIGLU || TN == 4, "SwiGLU pairs channel c with c + 32");
-  static_assert(FMT == SMOE_BF16 || FMT == SMOE_FP8_E4M3, "int4: k_gemm_stream4");
-  __shared__ __attribute__((aligned(1024))) uint8_t ring[NS * STAGE];
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int q = lane >> 4, l16 = lane & 15;
-  // (group, strip) of this workgroup: workgroup ids are dealt to the 8 XCDs
-  // round robin, so the linear id is split into 8 contiguous ranges of
-  // (group, strip) pairs, one per XCD, and a group's strips share one L2
-  // (its activation rows come from HBM once instead of once per strip)
-  int g, nb;
-  {
-    const int S = gridDim.x, T = S * gridDim.y;
-    const int bid = blockIdx.x + S * blockIdx.y;
-    const int x = bid & 7, local = bid >> 3, base = T >> 3, rem = T & 7;
-    const int logical = x * base + min(x, rem) + local;
-    g = logical / S;
-    nb = (logical - g * S) * 256;
-  }
-  int r_lo, r_hi;
-  if (p.G == 0) {
-    r_lo = 0;
-    r_hi = p.single_rows;
-  } else {
-    r_lo = p.grp_off[g];
-    r_hi = p.grp_off[g + 1];
-  }
-  if (r_hi <= r_lo) return;  // workgroup-uniform, before any barrier
-  const int KC = p.K / 64;
-  // weight DMA: instruction j of wave w fills bytes [(4 j + w) KB, +1 KB) of
-  // the stage's weight region; lane l writes byte b = that + 16 l, i.e. row
-  // b / WB, physical chunk (b % WB) / 16 (which holds the logical chunk the
-  // swizzle maps there)
-  const uint8_t* wsrc[W_LD];
-#pragma unroll
-  for (int j = 0; j < W_LD; ++j) {
-    const int b = (4 * j + wave) * 1024 + 16 * lane;
-    const int row = b / WB, pc = (b % WB) >> 4;
-    const int lc = sw_chunk<CPR>(row, pc);  // the map is an involution
-    const int n = min(nb + row, p.N_out - 1);  // channels past N_out: loaded, never stored
-    wsrc[j] = reinterpret_cast<const uint8_t*>(p.W) +
-              (g * p.w_gstride + static_cast<int64_t>(n) * p.ldw) * ESZ2 / 2 + lc * 16;
-  }
-  const uint16_t* A = reinterpret_cast<const uint16_t*>(p.A);
-  for (int m0 = r_lo; m0 < r_hi; m0 += ROWS) {  // passes (uniform)
-    // activation DMA: instruction j of wave w covers rows 8 (4 j + w) .. +8,
-    // lane l: row + l / 8, physical chunk l % 8
-    const uint16_t* asrc[A_LD];
-#pragma unroll
-    for (int j = 0; j < A_LD; ++j) {
-      const int r = 8 * (4 * j + wave) + (lane >> 3);
-      const int pr = m0 + r < r_hi ? m0 + r : r_lo;  // rows past the group: valid, never stored
-      const int ar = p.a_rows ? p.a_rows[pr] : pr;
-      asrc[j] = A + static_cast<int64_t>(ar) * p.lda + (sw_chunk<8>(r, lane & 7) << 3);
-    }
-    auto issue = [&](int kc) {  // DMA of chunk kc into ring slot kc % NS
-      uint8_t* base = ring + (kc % NS) * STAGE;
-#pragma unroll
-      for (int j = 0; j < W_LD; ++j)
-        __builtin_amdgcn_global_load_lds((gbl_vptr)(wsrc[j] + static_cast<int64_t>(kc) * WB),
-                                         (lds_vptr)(base + (4 * j + wave) * 1024), 16, 0, 0);
-#pragma unroll
-      for (int j = 0; j < A_LD; ++j)
-        __builtin_amdgcn_global_load_lds((gbl_vptr)(asrc[j] + kc * 64),
-                                         (lds_vptr)(base + W_BYTES + (4 * j + wave) * 1024), 16,
-                                         0, 0);
-    };
-    f32x4 acc[TN][RT];
-#pragma unroll
-    for (int t = 0; t < TN; ++t)
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) acc[t][rt] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    // prologue: chunks 0 .. NS-2 in flight, chunk 0 landed everywhere
-#pragma unroll
-    for (int st = 0; st < NS - 1; ++st)
-      if (st < KC) issue(st);
-    if (KC >= NS - 1) wait_vmcnt<(NS - 2) * LD>();
-    else wait_vmcnt<0>();
-    wait_lgkm0();  // the scale table (int4) is written
-    __builtin_amdgcn_s_barrier();
-    for (int kc = 0; kc < KC; ++kc) {
-      if (kc > 0) {
-        // own part of chunk kc landed (kc+1 .. kc+NS-2 may fly); chunk kc-1
-        // is no longer read by anyone after the barrier
-        if (kc + NS - 2 < KC) wait_vmcnt<(NS - 2) * LD>();
-        else wait_vmcnt<0>();
-        wait_lgkm0();
-        __builtin_amdgcn_s_barrier();
-      }
-      if (kc + NS - 1 < KC) issue(kc + NS - 1);  // into the slot chunk kc-1 used
-      const uint8_t* sw = ring + (kc % NS) * STAGE;
-      const uint8_t* sa = sw + W_BYTES;
-      bf16x8 wlo[TN], whi[TN];
-#pragma unroll
-      for (int t = 0; t < TN; ++t) {
-        const int row = wave * 64 + t * 16 + l16;
-        WRaw<FMT> r;
-        if constexpr (FMT == SMOE_BF16) {
-          r.a = *reinterpret_cast<const u32x4*>(sw + row * WB + (sw_chunk<CPR>(row, 2 * q) << 4));
-          r.b = *reinterpret_cast<const u32x4*>(sw + row * WB + (sw_chunk<CPR>(row, 2 * q + 1) << 4));
-        } else {
-          r.a = *reinterpret_cast<const u32x4*>(sw + row * WB + (sw_chunk<CPR>(row, q) << 4));
-        }
-        skinny_wconv<FMT>(r, wlo[t], whi[t]);
-      }
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
-        const int r = rt * 16 + l16;
-        const bf16x8 blo = *reinterpret_cast<const bf16x8*>(sa + r * 128 + (sw_chunk<8>(r, 2 * q) << 4));
-        const bf16x8 bhi = *reinterpret_cast<const bf16x8*>(sa + r * 128 + (sw_chunk<8>(r, 2 * q + 1) << 4));
-#pragma unroll
-        for (int t = 0; t < TN; ++t) {
-          acc[t][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wlo[t], blo, acc[t][rt], 0, 0, 0);
-          acc[t][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(whi[t], bhi, acc[t][rt], 0, 0, 0);
-        }
-      }
-    }
-    // lane: channels nb + 64 wave + 16 t + 4 q + (0..3) of row m0 + 16 rt + l16
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      const int row = m0 + rt * 16 + l16;
-      if (row >= r_hi) continue;
-#pragma unroll
-      for (int t = 0; t < TN; ++t) {
-        const int c = nb + wave * 64 + 16 * t + 4 * q;
-        if (c >= p.N_out) continue;
-        if constexpr (EPI == EPI_SWIGLU) {
-          if (t >= 2) continue;
-          const f32x4 v = acc[t][rt], up = acc[t + 2][rt];
-          const int u0 = (c >> 6) * 32 + (c & 31);
-          float o[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float gs = v[i] * col_scale(p, FMT, g, c + i);
-            const float us = up[i] * col_scale(p, FMT, g, c + 32 + i) + bias_at(p, g, u0 + i);
-            o[i] = silu(gs) * us;
-          }
-          const int64_t off = static_cast<int64_t>(row) * p.ldo + u0;
-          if (p.out_dtype == SMOE_F32)
-            *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.out) + off) = f32x4{o[0], o[1], o[2], o[3]};
-          else
-            *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(p.out) + off) =
-                u32x2{pack_bf2(o[0], o[1]), pack_bf2(o[2], o[3])};
-        } else {
-          store4<EPI>(p, FMT, g, row, c, acc[t][rt]);
-        }
-      }
-    }
-    if (m0 + ROWS < r_hi) {  // another pass: every wave is done with the ring
-      wait_lgkm0();
-      __builtin_amdgcn_s_barrier();
-    }
-  }
-}
-
-// int4 weights at the stream kernel's row counts, with the dequant beside
-// the MFMAs instead of before them: inside a chunk the 16 weights of tile
-// t+1 are widened (about 3 VALU operations per weight) in the same stretch
-// of code as tile t's MFMAs, so the VALU and the matrix pipe of a wave work
-// side by side; only tile 0's widening is exposed.  The activation
+//
+// The dequant runs beside the MFMAs instead of before them: inside a chunk
+// the 16 weights of tile t+1 are widened (about 3 VALU operations per weight)
+// in the same stretch of code as tile t's MFMAs, so the VALU and the matrix
+// pipe of a wave work side by side; only tile 0's widening is exposed.  (The
+// tiles of smoe_gemm_mid.hip widen in front of their MFMAs, 64 rows at a time:
+// 72 us against 60 at 64 groups of 68 rows, 2048 -> 1408.)  The activation
 // fragments of all live row tiles are read once per chunk.  The number of
 // live 16-row tiles of a pass is a template parameter (one instantiation per
 // count, chosen per pass), so tiles past the group's last row issue neither
 // MFMAs nor activation DMA, and the loop body has no branches to split it.
-// Waves whose channels all lie past N_out skip the arithmetic.  Work
-// split, ring, swizzles and XCD-aware workgroup order are those
-// of k_gemm_stream; the strip's group scales sit in an LDS table after the
-// ring, in the same LDS object (with a second LDS object the compiler waits
-// for every outstanding DMA before reads of the table, draining the ring's
-// prefetch).  A wave owns TN 16-channel tiles (a strip of 64 TN channels);
-// it brings its own channels' weights into the ring, WWB bytes per chunk in
-// 1 KB DMA instructions, the last one on the lanes it needs when TN is odd.
-// TN only decides which channels a wave holds: every output is summed in the
-// same order, so the bits do not depend on it.
+// Waves whose channels all lie past N_out skip the arithmetic.  The linear
+// workgroup id is split into 8 contiguous ranges of (group, strip), one per
+// XCD, so a group's strips share one L2.  The strip's group scales sit in an
+// LDS table after the ring, in the same LDS object (with a second LDS object
+// the compiler waits for every outstanding DMA before reads of the table,
+// draining the ring's prefetch).  A wave brings its own channels' weights
+// into the ring, WWB bytes per chunk in 1 KB DMA instructions, the last one
+// on the lanes it needs when TN is odd.  TN only decides which channels a
+// wave holds: every output is summed in the same order, so the bits do not
+// depend on it.
+constexpr int kStreamScaleMax = 4096;  // int4 scale-table entries per strip
+
 template <int EPI, int RT, int NS = 3, int TN = 4>
 __global__ __launch_bounds__(256, 2) void k_gemm_stream4(const GemmArgs p) {
   constexpr int WB = 32, CPR = 2;  // int4: 32 B per channel per 64-k chunk
@@ -2351,20 +1895,6 @@ int launch_skinny(const GemmArgs& a, hipStream_t s) {
   }
 }
 
-template <int FMT, int RT, int NS, int WGS>
-int launch_stream_fmt(const GemmArgs& a, hipStream_t s) {
-  const dim3 grid((a.N_out + 255) / 256, a.G == 0 ? 1 : a.G), block(256);
-  switch (a.epi) {
-    case EPI_F32_BIAS: SMOE_LAUNCH((k_gemm_stream<FMT, EPI_F32_BIAS, RT, NS, WGS>), grid, block, 0, s, a); break;
-    case EPI_ROWSCALE: SMOE_LAUNCH((k_gemm_stream<FMT, EPI_ROWSCALE, RT, NS, WGS>), grid, block, 0, s, a); break;
-    case EPI_GELU: SMOE_LAUNCH((k_gemm_stream<FMT, EPI_GELU, RT, NS, WGS>), grid, block, 0, s, a); break;
-    case EPI_SWIGLU: SMOE_LAUNCH((k_gemm_stream<FMT, EPI_SWIGLU, RT, NS, WGS>), grid, block, 0, s, a); break;
-    case EPI_DOWN: SMOE_LAUNCH((k_gemm_stream<FMT, EPI_DOWN, RT, NS, WGS>), grid, block, 0, s, a); break;
-    default: return SMOE_EINVAL;
-  }
-  return hipGetLastError() == hipSuccess ? SMOE_OK : SMOE_EHIP;
-}
-
 template <int RT, int NS = 3, int TN = 4>
 int launch_stream4(const GemmArgs& a, hipStream_t s) {
   const dim3 grid((a.N_out + 64 * TN - 1) / (64 * TN), a.G == 0 ? 1 : a.G), block(256);
@@ -2402,30 +1932,15 @@ int stream4_tn(const GemmArgs& a) {
   return cost(3) < cost(4) ? 3 : 4;
 }
 
-// Two workgroups per CU (one's dequant and waits overlap the other's MFMAs):
-// LDS per workgroup int4 3 x 20 KB + 16 KB scales, fp8 3 x 24 KB (64-row
-// passes), bf16 3 x 40 KB (one workgroup per CU).
-int launch_stream(const GemmArgs& a, hipStream_t s) {
-  switch (a.fmt) {
-    case SMOE_BF16: return launch_stream_fmt<SMOE_BF16, 4, 3, 1>(a, s);
-    case SMOE_FP8_E4M3: return launch_stream_fmt<SMOE_FP8_E4M3, 4, 3, 2>(a, s);
-    case SMOE_INT4:
-      if (256 * (a.K / a.group_size) > kStreamScaleMax || (a.group_size & (a.group_size - 1)))
-        return SMOE_EUNSUPPORTED;
-      return stream4_tn(a) == 3 ? launch_stream4<6, 3, 3>(a, s) : launch_stream4<6>(a, s);
-    default: return SMOE_EUNSUPPORTED;
-  }
-}
-
-// Whether the weight-streaming kernels can take the GEMM: every 16-byte
-// (int4: 8-byte) load they issue aligned, K in 64-wide steps.
-bool stream_aligned(const GemmArgs& a) {
-  if (a.K % 64 || a.N_out % 4 || a.ldo % 4 || a.lda % 8) return false;
-  const int walign = a.fmt == SMOE_BF16 ? 8 : 16;  // elements per aligned load
-  if (a.ldw % walign || a.w_gstride % walign) return false;
-  if (a.fmt == SMOE_INT4 && a.group_size % 16) return false;
-  if (a.bias && a.bias_gstride % 4) return false;  // 16-byte bias loads (int4 epilogue)
-  return a.fmt == SMOE_BF16 || a.fmt == SMOE_FP8_E4M3 || a.fmt == SMOE_INT4;
+// Whether the int4 stream kernel takes the GEMM: every 16-byte (weights and
+// activations) load it issues aligned, K in 64-wide steps, the strip's scales
+// within its LDS table.  Two workgroups per CU (one's dequant and waits
+// overlap the other's MFMAs): LDS per workgroup 3 x 20 KB + 16 KB scales.
+bool stream4_fits(const GemmArgs& a) {
+  if (a.fmt != SMOE_INT4 || a.K % 64 || a.N_out % 4 || a.ldo % 4 || a.lda % 8) return false;
+  if (a.ldw % 16 || a.w_gstride % 16 || a.group_size % 16) return false;
+  if (a.bias && a.bias_gstride % 4) return false;  // 16-byte bias loads
+  return 256 * (a.K / a.group_size) <= kStreamScaleMax && !(a.group_size & (a.group_size - 1));
 }
 
 // Whether every 16-byte (int4: 8-byte) load the skinny kernel issues is
@@ -2577,16 +2092,10 @@ int launch_grouped_gemm(const GemmArgs& a, hipStream_t s) {
     if (a.G > 0 && a.epi != EPI_SWIGLU && a.N_out <= 64 && rpg > 8) return launch_skinny<2, 2>(a, s);
     return rpg <= 8 || a.G == 0 ? launch_skinny<4, 1>(a, s) : launch_skinny<4, 2>(a, s);
   }
-  // a few dozen to 128 rows per group (mixed decode + prefill): one
-  // workgroup per (group, 256-channel strip) over all the group's rows,
-  // weights and activations streamed through an LDS ring
-  {
-    const int rpg = a.G == 0 ? a.single_rows : a.max_rows / a.G;
-    if (a.G > 0 && rpg <= 128 && a.N_out >= 128 && stream_aligned(a) &&
-        (a.fmt != SMOE_INT4 || (256 * (a.K / a.group_size) <= kStreamScaleMax &&
-                                (a.group_size & (a.group_size - 1)) == 0)))
-      return launch_stream(a, s);
-  }
+  // int4, a few dozen to 128 rows per group (mixed decode + prefill): one
+  // workgroup per (group, channel strip) over all the group's rows
+  if (a.G > 0 && a.max_rows / a.G <= 128 && a.N_out >= 128 && stream4_fits(a))
+    return stream4_tn(a) == 3 ? launch_stream4<6, 3, 3>(a, s) : launch_stream4<6>(a, s);
   // large bf16 / fp8 (tile copy) problems (K % 64): 256 x 256 tiles, 8 waves in two ping-pong
   // groups when N_out % 256 == 0 (128-row tiles, two workgroups per CU, for
   // groups of a few hundred rows); otherwise 256 x 128 ring tiles, two
@@ -2608,6 +2117,9 @@ int launch_grouped_gemm(const GemmArgs& a, hipStream_t s) {
     }
     if (a.N_out % 128 == 0 && a.fmt == SMOE_BF16) return launch_ring<128, 3, 4>(a, s);
   }
+  // what is left of the wide outputs: up to 255 rows per group, f32 results,
+  // fp8 / int4 without a tile copy
+  if (gemm_mid_fits(a)) return launch_gemm_mid(a, s);
   const bool b64 = bk == 64;
   // narrow outputs (router / edge logits, N_out = E): 64-row tiles, one
   // 16-row MFMA strip per wave, so the grid has enough workgroups

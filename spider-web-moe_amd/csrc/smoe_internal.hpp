@@ -101,6 +101,10 @@ int launch_grouped_gemm(const GemmArgs& a, hipStream_t s);
 bool gemm_f32_fits(const GemmArgs& a);
 int launch_gemm_f32(const GemmArgs& a, hipStream_t s);
 int launch_gemm_f32_front(const GemmArgs& a, hipStream_t s);  // W2: launch_front_dense
+// bf16 / fp8 / int4 GEMMs of a few dozen to a few hundred rows per group
+// (smoe_gemm_mid.hip): K % 64 == 0, N_out >= 128, 16-byte operand rows and stores
+bool gemm_mid_fits(const GemmArgs& a);
+int launch_gemm_mid(const GemmArgs& a, hipStream_t s);
 // true when launch_grouped_gemm runs `a` on a ping-pong kernel, which reads
 // At and writes out_tiles (the fields themselves are ignored here)
 bool gemm_takes_row_tiles(const GemmArgs& a);

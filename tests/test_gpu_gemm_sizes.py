@@ -64,3 +64,112 @@ def test_f32_grouped_tile_edges(n, h, u, e, k):
     up_err = (2 * h + 2) * 2.0 ** -24 * 4 * h ** 0.5 + 2e-7
     bound = (2 * u + 8) * 2.0 ** -24 * mag + up_err * u ** 0.5 * wt.sum(-1, keepdim=True).double()
     assert bool(((y - ref).abs() <= bound).all())
+
+
+# 33-255 rows per group on average, and any row count of fp8 / int4 without
+# tile copies: groups of 0, 1, 64, 65, .. rows (tiles of 64 and 128 rows), K
+# of one to five 64-k stages and channels off the 128-wide strips; 139 rows
+# per group on average: (192, 320) makes fewer 64 x 128 tiles than CUs (64 x
+# 64 tiles), (128, 2696) more (3 stages), (64, 5312) more than two per CU (2
+# stages), (128, 456) a partial strip; a third of the rows, (128, 2696): the
+# 64-row SwiGLU tiles
+@pytest.mark.parametrize("h,u,part", [(192, 320, 1), (128, 2696, 1), (64, 5312, 1), (128, 456, 1),
+                                      (128, 2696, 3)])
+@pytest.mark.parametrize("fmt,act", [("bf16", "gelu"), ("bf16", "swiglu"), ("fp8", "gelu"),
+                                     ("fp8", "swiglu"), ("int4", "gelu"), ("int4", "swiglu")])
+def test_grouped_mid_rows(fmt, act, h, u, part):
+    from spider_moe_amd import _native as n8
+    from spider_moe_amd.quant import (interleave_gate_up, interleave_gate_up_rows,
+                                      quantize_fp8_per_channel, quantize_int4)
+    from test_gpu_kernels import _experts_struct, _run_delta
+    # the down product's K is u: whole 64-k stages, or (2696, 456) bf16 on the
+    # vector kernel; fp8 needs 32-k and int4 whole scale groups
+    if u % 64 and (fmt != "bf16" or act == "swiglu"):
+        u += -u % 64
+    say("grouped mid", fmt, act, h, u, part)
+    g = torch.Generator().manual_seed(h + u)
+    rows = [r // part for r in (0, 3, 64, 65, 260, 300, 129, 300)]
+    e, n = len(rows), sum(rows)
+    idx = torch.cat([torch.full((r,), x, dtype=torch.int32) for x, r in enumerate(rows)])
+    idx = idx[torch.randperm(n, generator=g)].view(n, 1)
+    w = torch.rand(n, 1, generator=g) + 0.1
+    x = torch.randn(n, h, generator=g).to(torch.bfloat16)
+    nup = 2 * u if act == "swiglu" else u
+    mats = [torch.randn(e, nup, h, generator=g) * h ** -0.5, torch.randn(e, h, u, generator=g) * u ** -0.5]
+    bu, bd = torch.randn(e, u, generator=g) * 0.1, torch.randn(e, h, generator=g) * 0.1
+    vals, dev_w, dev_s, kw = [], [], [], {}
+    for i, m in enumerate(mats):
+        pair = act == "swiglu" and i == 0
+        if fmt == "bf16":
+            q, s = m.to(torch.bfloat16), None
+            vals.append(q.double())
+        elif fmt == "fp8":
+            q, s = quantize_fp8_per_channel(m)
+            q = q.view(torch.float8_e4m3fn)
+            vals.append(q.float().double() * s.view(e, -1, 1).double())
+            q, s = q.view(torch.uint8), s.view(e, -1).float()
+        else:
+            p4 = quantize_int4(m, 64, torch.float16)
+            q, s = p4.packed, p4.scales
+            b = q.view(torch.uint8).int()
+            nib = torch.stack([b & 15, b >> 4], -1).view(m.shape)
+            nib = torch.where(nib > 7, nib - 16, nib).float()
+            # the kernels multiply bf16(q * scale)
+            vals.append((nib * s.float().repeat_interleave(64, -1)).to(torch.bfloat16).double())
+        dev_w.append((interleave_gate_up(q[:, :u], q[:, u:]) if pair else q).contiguous().to(dev))
+        if s is not None and fmt == "fp8":
+            s = interleave_gate_up_rows(s[:, :u], s[:, u:]) if pair else s
+        elif s is not None:
+            s = interleave_gate_up(s[:, :u], s[:, u:]) if pair else s
+        dev_s.append(None if s is None else s.contiguous().to(dev))
+    if fmt != "bf16":
+        kw = dict(s_up=dev_s[0], s_down=dev_s[1], scale_dtype=n8.F16 if fmt == "int4" else n8.F32)
+    if fmt == "int4":
+        kw["group"] = 64
+    bu_d, bd_d = bu.to(dev), bd.to(dev)
+    code = {"bf16": n8.BF16, "fp8": n8.FP8_E4M3, "int4": n8.INT4}[fmt]
+    ex = _experts_struct(n8, code, n8.ACT_SWIGLU if act == "swiglu" else n8.ACT_GELU, e, h, u, *dev_w,
+                         b_up=bu_d, b_down=bd_d, **kw)
+    y = _run_delta(n8, ex, x.to(dev), idx.to(dev), w.to(dev)).double()
+    xd = x.double()
+    for i in range(e):
+        r = (idx[:, 0] == i).nonzero().squeeze(-1)
+        if not len(r):
+            continue
+        up = xd[r] @ vals[0][i].t()
+        if act == "swiglu":
+            a = torch.nn.functional.silu(up[:, :u]) * (up[:, u:] + bu[i].double())
+        else:
+            a = torch.nn.functional.gelu(up + bu[i].double())
+        wt = w[r].double()
+        ref = (a @ vals[1][i].t() + bd[i].double()) * wt
+        mag = (a.abs() @ vals[1][i].abs().t() + bd[i].abs().double()) * wt
+        # bf16 activations and rows: 2^-9 of each product and of the result;
+        # f32 sums of u and h terms and the f32 activation functions: far below
+        bound = (2.0 ** -9 + (2 * u + 2 * h) * 2.0 ** -24 + 1e-5) * mag + 2.0 ** -9 * ref.abs() + 1e-6
+        bad = (y[r] - ref).abs() > 1.01 * bound
+        assert not bool(bad.any()), (i, float(((y[r] - ref).abs() / bound).max()))
+
+
+# one group: f32 results (16-byte stores), fp8 codes on a bf16 input, K tails
+# and channels not a multiple of 4 (the general kernel)
+@pytest.mark.parametrize("n,k,n_out", [(65, 64, 128), (130, 320, 132), (500, 2816, 1024), (129, 192, 130),
+                                       (200, 96, 256), (2100, 128, 2052)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_linear_mid_rows(n, k, n_out, fp8):
+    from spider_moe_amd.forge import ForgeConfig, ForgeGEMM
+    from spider_moe_amd.quant import quantize_fp8_per_tensor
+    say("linear mid", n, k, n_out, fp8)
+    g = torch.Generator().manual_seed(n + k + n_out)
+    x = torch.randn(n, k, generator=g).to(torch.bfloat16)
+    w = (torch.randn(n_out, k, generator=g) * k ** -0.5).to(torch.bfloat16)
+    b = torch.randn(n_out, generator=g).to(torch.bfloat16)
+    y = ForgeGEMM(ForgeConfig(gemm_fp8=fp8)).linear(x.to(dev), w.to(dev), b.to(dev)).cpu().double()
+    wv = w.double()
+    if fp8:
+        codes, scale = quantize_fp8_per_tensor(w)
+        wv = codes.view(torch.float8_e4m3fn).float().double() * scale.double()
+    ref = x.double() @ wv.t() + b.double()
+    # f32 sums of k products, the result rounded to bf16
+    bound = 2.0 ** -8 * ref.abs() + (2 * k + 4) * 2.0 ** -24 * (x.abs().double() @ wv.abs().t() + b.abs().double())
+    assert bool(((y - ref).abs() <= bound).all())

@@ -98,7 +98,8 @@ typedef struct smoe_experts {
    * of them by the decode weight stream and the ping-pong GEMM (bit-identical
    * results for bf16).  int4 (smoe_pack_int4_qtiles): the int4 tile layout,
    * read by the ping-pong GEMM at prefill sizes (>= 256 rows per expert) in
-   * place of the general int4 kernel; the decode and stream kernels keep
+   * place of the general int4 kernel, and by the decode weight stream for
+   * group sizes that are powers of two from 64; the kernels between them keep
    * reading the packed int4. */
   const void* w_up_tiles;
   const void* w_down_tiles;

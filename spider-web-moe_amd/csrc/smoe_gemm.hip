@@ -829,16 +829,25 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_skinny(const GemmArgs p) {
 // waves of the grid would do their arithmetic at the end).  The KSPLIT waves
 // of a slice add their partial sums through LDS in wave order (bit-identical
 // run to run); with KSPLIT 1 no wave waits for another.  k order inside a
-// 64-wide step, the same for both operands: bf16 weights take k 8q..8q+7
-// (first MFMA) and 32+8q.. (second), so each of their two 16-byte loads
-// covers 64 contiguous bytes of 16 rows; fp8 / int4 take the 16 consecutive
-// k at 16q.  Only the last 2D - 1 steps' refills sit under a branch, so the
+// 64-wide step, the same for both operands: bf16 weights and int4 tiles take
+// k 8q..8q+7 (first MFMA) and 32+8q.. (second), so each of a bf16 step's two
+// 16-byte loads covers 64 contiguous bytes of 16 rows; fp8 and row-major int4
+// take the 16 consecutive k at 16q.  Only the last 2D - 1 steps' refills sit under a branch, so the
 // main loop's waits count the loads in flight exactly.
+//
+// int4: a scale converted (or its type chosen) where it is loaded waits for
+// that load, and with it for every load before it, so the ring holds the bits
+// and the type is a template parameter; the row-major codes are 32 bytes of
+// each of 64 rows per step, a quarter of a cache line, the tile layout's 2 KB
+// contiguous.  64 experts, 16 tokens top-2 (36 MB of codes), us per launch:
+// up 2048 -> 1408 33.5 -> 31.5 (bits) -> 23.9 (tiles), down 32.8 -> 22.3 -> 18.2
+// (2 TB/s; the lookup and the first loads' round trips are half of that; a
+// ring of 6 steps 26.3 and 19.0).
 template <int FMT>
 struct DRaw;
 template <> struct DRaw<SMOE_BF16> { u32x4 a, b; };
 template <> struct DRaw<SMOE_FP8_E4M3> { u32x4 a; };
-template <> struct DRaw<SMOE_INT4> { u32x2 a; float s; };
+template <> struct DRaw<SMOE_INT4> { u32x2 a; uint32_t s; };  // s: the scale's bits (f16 or f32)
 
 // The position of the j-th set bit (0-based) of m; j < popcount(m).
 __device__ __forceinline__ int nth_set_bit(uint64_t m, int j) {
@@ -873,13 +882,15 @@ __host__ __device__ __forceinline__ bool decode_spec(const GemmArgs& p) {
 // found from the front's selections by a ballot over the tokens (lane t);
 // its weights are known before any load.  red: LDS of
 // (KSPLIT > 1 ? 4 : 1) * TNW * RT * 64 f32x4.
-template <int FMT, int EPI, int TNW, int RT, int KSPLIT, int D, bool PK, bool SEL>
+template <int FMT, int EPI, int TNW, int RT, int KSPLIT, int D, bool PK, bool SEL, bool SF16 = false>
 __device__ __forceinline__ void decode_gemm(const GemmArgs& p, int gy, f32x4* red) {
   constexpr int ESZ2 = FMT == SMOE_BF16 ? 4 : (FMT == SMOE_FP8_E4M3 ? 2 : 1);  // 2 x bytes/elt
   constexpr int CS = 4 / KSPLIT;  // channel slices per workgroup
   static_assert(4 % KSPLIT == 0, "KSPLIT divides the 4 waves");
   static_assert(EPI != EPI_SWIGLU || TNW == 2 || TNW == 4, "SwiGLU slices pair gate and up tiles");
-  static_assert(!PK || FMT != SMOE_INT4, "the weight tile layout holds bf16 or fp8 weights");
+  static_assert(!PK || FMT != SMOE_INT4 || TNW == 4, "an int4 tile block holds 64 channels");
+  constexpr bool PK4 = PK && FMT == SMOE_INT4;
+  constexpr bool K32 = FMT == SMOE_BF16 || PK4;  // a step's MFMAs take its lower / upper 32 k
   static_assert(!SEL || EPI == EPI_ROWSCALE, "row selection: the edge projection");
   constexpr int BLK = 512 * ESZ2;  // bytes of one 64-k step of a 16-row tile
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -949,19 +960,31 @@ __device__ __forceinline__ void decode_gemm(const GemmArgs& p, int gy, f32x4* re
                                     16 * (t % (TNW / 2)) + 32 * (t / (TNW / 2))
                               : 16 * (TNW * slice + t);
   const uint8_t* wrow[TNW];
-  int wn[TNW];
+  const uint8_t* srow[TNW];  // int4: the channel's group scales
 #pragma unroll
   for (int t = 0; t < TNW; ++t) {
     const int n = min(c0[t] + l16, p.N_out - 1);
-    wn[t] = n;
     wrow[t] = reinterpret_cast<const uint8_t*>(p.W) +
               (g * p.w_gstride + static_cast<int64_t>(n) * p.ldw) * ESZ2 / 2;
+    if constexpr (FMT == SMOE_INT4)
+      srow[t] = reinterpret_cast<const uint8_t*>(p.S) +
+                (g * p.s_gstride + static_cast<int64_t>(n) * (p.K / p.group_size)) * (SF16 ? 2 : 4);
   }
   // weight tile layout: tile t's 64-k step st is block (g * N_out/16 + t) *
   // K/64 + st of BLK bytes, lane l's fragments at 16 l (fp8: 64 k) or at
-  // 16 l and 1 KB + 16 l (bf16: k 8q.. and 32 + 8q..)
+  // 16 l and 1 KB + 16 l (bf16: k 8q.. and 32 + 8q..).  int4 tile layout: the
+  // slice's 64 channels x 32 k are one block of 1 KB, tile t's codes of lane l
+  // (k 8q..) at 256 t + 4 l, blocks consecutive in k
   const uint8_t* wtile[TNW];
-  if constexpr (PK) {
+  int gs_shift = 0;
+  if constexpr (PK4) {
+    gs_shift = 31 - __builtin_clz(p.group_size);
+    const int quad = min(slice, (p.N_out >> 6) - 1);
+#pragma unroll
+    for (int t = 0; t < TNW; ++t)
+      wtile[t] = reinterpret_cast<const uint8_t*>(p.Wt) +
+                 ((static_cast<int64_t>(g) * (p.N_out >> 6) + quad) * (p.K >> 5) << 10) + 256 * t + 4 * lane;
+  } else if constexpr (PK) {
 #pragma unroll
     for (int t = 0; t < TNW; ++t) {
       const int tile = min(c0[t], p.N_out - 16) >> 4;
@@ -979,7 +1002,14 @@ __device__ __forceinline__ void decode_gemm(const GemmArgs& p, int gy, f32x4* re
     const int k0 = 64 * min(s_begin + i, last);
 #pragma unroll
     for (int t = 0; t < TNW; ++t) {
-      if constexpr (PK) {
+      if constexpr (PK4) {
+        const uint8_t* blk = wtile[t] + (static_cast<int64_t>(k0 >> 5) << 10);
+        wr[d][t].a.x = *reinterpret_cast<const uint32_t*>(blk);
+        wr[d][t].a.y = *reinterpret_cast<const uint32_t*>(blk + 1024);
+        const int gi = k0 >> gs_shift;
+        if constexpr (SF16) wr[d][t].s = reinterpret_cast<const uint16_t*>(srow[t])[gi];
+        else wr[d][t].s = reinterpret_cast<const uint32_t*>(srow[t])[gi];
+      } else if constexpr (PK) {
         const uint8_t* blk = wtile[t] + static_cast<int64_t>(k0 >> 6) * BLK;
         wr[d][t].a = *reinterpret_cast<const u32x4*>(blk);
         if constexpr (FMT == SMOE_BF16) wr[d][t].b = *reinterpret_cast<const u32x4*>(blk + 1024);
@@ -989,12 +1019,12 @@ __device__ __forceinline__ void decode_gemm(const GemmArgs& p, int gy, f32x4* re
       } else if constexpr (FMT == SMOE_FP8_E4M3) {
         wr[d][t].a = *reinterpret_cast<const u32x4*>(wrow[t] + k0 + 16 * q);
       } else {
-        const int k = k0 + 16 * q;
+        const int k = k0 + 16 * q, gi = k / p.group_size;
         wr[d][t].a = *reinterpret_cast<const u32x2*>(wrow[t] + (k >> 1));
-        wr[d][t].s = load_scale(p.S,
-                                g * p.s_gstride + static_cast<int64_t>(wn[t]) * (p.K / p.group_size) +
-                                    k / p.group_size,
-                                p.s_f16);
+        // the bits only: a conversion here would wait for this load, and with
+        // it for every load before it
+        if constexpr (SF16) wr[d][t].s = reinterpret_cast<const uint16_t*>(srow[t])[gi];
+        else wr[d][t].s = reinterpret_cast<const uint32_t*>(srow[t])[gi];
       }
     }
   };
@@ -1002,7 +1032,7 @@ __device__ __forceinline__ void decode_gemm(const GemmArgs& p, int gy, f32x4* re
     const int k0 = 64 * min(s_begin + i, last);
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-      if constexpr (FMT == SMOE_BF16) {
+      if constexpr (K32) {
         av[d][rt][0] = *reinterpret_cast<const u32x4*>(arow[rt] + k0 + 8 * q);
         av[d][rt][1] = *reinterpret_cast<const u32x4*>(arow[rt] + k0 + 32 + 8 * q);
       } else {
@@ -1054,8 +1084,11 @@ __device__ __forceinline__ void decode_gemm(const GemmArgs& p, int gy, f32x4* re
         l = u32x4{a0.x, a0.y, a1.x, a1.y};
         h = u32x4{b0.x, b0.y, b1.x, b1.y};
       } else {
-        l = int4x8_to_bf16x8(wr[d][t].a.x, wr[d][t].s);
-        h = int4x8_to_bf16x8(wr[d][t].a.y, wr[d][t].s);
+        const float sc = SF16 ? static_cast<float>(__builtin_bit_cast(
+                                    _Float16, static_cast<uint16_t>(wr[d][t].s)))
+                              : __uint_as_float(wr[d][t].s);
+        l = int4x8_to_bf16x8(wr[d][t].a.x, sc);
+        h = int4x8_to_bf16x8(wr[d][t].a.y, sc);
       }
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
@@ -1192,10 +1225,10 @@ __device__ __forceinline__ void decode_gemm(const GemmArgs& p, int gy, f32x4* re
   else emit(std::false_type{});
 }
 
-template <int FMT, int EPI, int TNW, int RT, int KSPLIT, int D, bool PK = false>
+template <int FMT, int EPI, int TNW, int RT, int KSPLIT, int D, bool PK = false, bool SF16 = false>
 __global__ __launch_bounds__(256) void k_gemm_decode(const GemmArgs p) {
   __shared__ f32x4 red[(KSPLIT > 1 ? 4 : 1) * TNW * RT * 64];
-  decode_gemm<FMT, EPI, TNW, RT, KSPLIT, D, PK, false>(p, blockIdx.y, red);
+  decode_gemm<FMT, EPI, TNW, RT, KSPLIT, D, PK, false, SF16>(p, blockIdx.y, red);
 }
 
 // The decode edge projection (bf16 weight tiles, row selection from the
@@ -1784,7 +1817,7 @@ int launch_simt(const GemmArgs& a, hipStream_t s) {
   return launch_simt_bn<64, 64, FMT>(a, s);
 }
 
-template <int FMT, int RT, int KSPLIT, bool PK>
+template <int FMT, int RT, int KSPLIT, bool PK, bool SF16>
 int launch_decode_fmt(const GemmArgs& a, hipStream_t s) {
   // one workgroup per (4 / KSPLIT slices of 64 channels, tile of 16*RT rows);
   // 3 steps in flight per wave
@@ -1795,22 +1828,26 @@ int launch_decode_fmt(const GemmArgs& a, hipStream_t s) {
   if (tiles == 0) return SMOE_OK;
   const int slices = (a.N_out + 16 * TNW - 1) / (16 * TNW);
   const dim3 grid((slices + CS - 1) / CS, tiles, 1);
+  auto go = [&](auto epi) {
+    SMOE_LAUNCH((k_gemm_decode<FMT, decltype(epi)::value, TNW, RT, KSPLIT, D, PK, SF16>), grid,
+                dim3(256), 0, s, a);
+    return hipGetLastError() == hipSuccess ? SMOE_OK : SMOE_EHIP;
+  };
   switch (a.epi) {
-    case EPI_F32_BIAS: SMOE_LAUNCH((k_gemm_decode<FMT, EPI_F32_BIAS, TNW, RT, KSPLIT, D, PK>), grid, dim3(256), 0, s, a); break;
-    case EPI_ROWSCALE: SMOE_LAUNCH((k_gemm_decode<FMT, EPI_ROWSCALE, TNW, RT, KSPLIT, D, PK>), grid, dim3(256), 0, s, a); break;
-    case EPI_GELU: SMOE_LAUNCH((k_gemm_decode<FMT, EPI_GELU, TNW, RT, KSPLIT, D, PK>), grid, dim3(256), 0, s, a); break;
-    case EPI_DOWN: SMOE_LAUNCH((k_gemm_decode<FMT, EPI_DOWN, TNW, RT, KSPLIT, D, PK>), grid, dim3(256), 0, s, a); break;
-    case EPI_SWIGLU: SMOE_LAUNCH((k_gemm_decode<FMT, EPI_SWIGLU, TNW, RT, KSPLIT, D, PK>), grid, dim3(256), 0, s, a); break;
+    case EPI_F32_BIAS: return go(std::integral_constant<int, EPI_F32_BIAS>{});
+    case EPI_ROWSCALE: return go(std::integral_constant<int, EPI_ROWSCALE>{});
+    case EPI_GELU: return go(std::integral_constant<int, EPI_GELU>{});
+    case EPI_DOWN: return go(std::integral_constant<int, EPI_DOWN>{});
+    case EPI_SWIGLU: return go(std::integral_constant<int, EPI_SWIGLU>{});
     default: return SMOE_EINVAL;
   }
-  return hipGetLastError() == hipSuccess ? SMOE_OK : SMOE_EHIP;
 }
 
-template <int FMT, int RT, bool PK = false>
+template <int FMT, int RT, bool PK = false, bool SF16 = false>
 int launch_decode_split(const GemmArgs& a, int ksplit, hipStream_t s) {
-  if (ksplit == 1) return launch_decode_fmt<FMT, RT, 1, PK>(a, s);
-  if (ksplit == 2) return launch_decode_fmt<FMT, RT, 2, PK>(a, s);
-  return launch_decode_fmt<FMT, RT, 4, PK>(a, s);
+  if (ksplit == 1) return launch_decode_fmt<FMT, RT, 1, PK, SF16>(a, s);
+  if (ksplit == 2) return launch_decode_fmt<FMT, RT, 2, PK, SF16>(a, s);
+  return launch_decode_fmt<FMT, RT, 4, PK, SF16>(a, s);
 }
 
 }  // namespace
@@ -1856,6 +1893,19 @@ int launch_decode(const GemmArgs& a, hipStream_t s) {
       return rt == 1 ? launch_decode_split<SMOE_FP8_E4M3, 1>(a, ksplit, s)
                      : launch_decode_split<SMOE_FP8_E4M3, 2>(a, ksplit, s);
     case SMOE_INT4:
+      // the int4 tile layout: 1 KB per 32-k step of a 64-channel slice instead
+      // of 32 bytes of each of 64 rows
+      if (a.Wt && a.N_out % 64 == 0 && a.group_size % 64 == 0 &&
+          (a.group_size & (a.group_size - 1)) == 0) {
+        if (a.s_f16)
+          return rt == 1 ? launch_decode_split<SMOE_INT4, 1, true, true>(a, ksplit, s)
+                         : launch_decode_split<SMOE_INT4, 2, true, true>(a, ksplit, s);
+        return rt == 1 ? launch_decode_split<SMOE_INT4, 1, true>(a, ksplit, s)
+                       : launch_decode_split<SMOE_INT4, 2, true>(a, ksplit, s);
+      }
+      if (a.s_f16)
+        return rt == 1 ? launch_decode_split<SMOE_INT4, 1, false, true>(a, ksplit, s)
+                       : launch_decode_split<SMOE_INT4, 2, false, true>(a, ksplit, s);
       return rt == 1 ? launch_decode_split<SMOE_INT4, 1>(a, ksplit, s)
                      : launch_decode_split<SMOE_INT4, 2>(a, ksplit, s);
     default: return SMOE_EUNSUPPORTED;

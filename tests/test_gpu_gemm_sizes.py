@@ -173,3 +173,66 @@ def test_linear_mid_rows(n, k, n_out, fp8):
     # f32 sums of k products, the result rounded to bf16
     bound = 2.0 ** -8 * ref.abs() + (2 * k + 4) * 2.0 ** -24 * (x.abs().double() @ wv.abs().t() + b.abs().double())
     assert bool(((y - ref).abs() <= bound).all())
+
+
+# decode steps on int4 experts with their tile copy: slices past N_out (H 192,
+# U 448), K split over 1, 2 and 4 waves (K 128, 448, 832), groups found by
+# lookup (fewer than two rows per expert on average) and directly, scales of
+# both types, one per 64 and 128 k
+@pytest.mark.parametrize("n,h,u,act", [(1, 192, 448, "gelu"), (7, 832, 128, "swiglu"), (9, 128, 832, "gelu"),
+                                       (40, 448, 192, "swiglu"), (100, 832, 448, "gelu")])
+@pytest.mark.parametrize("group,sdt", [(64, torch.float16), (64, torch.float32), (128, torch.float16)])
+def test_decode_int4_tiles(n, h, u, act, group, sdt):
+    from spider_moe_amd import _native as n8
+    from spider_moe_amd.quant import interleave_gate_up, quantize_int4
+    from test_gpu_kernels import _experts_struct, _run_delta
+    if h % group or u % group:
+        h, u = -(-h // group) * group, -(-u // group) * group
+    say("decode int4 tiles", n, h, u, act, group, sdt)
+    e, k = 8, 2
+    g = torch.Generator().manual_seed(n + h + u + group)
+    x = torch.randn(n, h, generator=g).to(torch.bfloat16)
+    idx = torch.stack([torch.randperm(e - 1, generator=g)[:k] for _ in range(n)]).to(torch.int32)
+    w = torch.rand(n, k, generator=g) + 0.1
+    nup = 2 * u if act == "swiglu" else u
+    vals, codes, tiles, scales = [], [], [], []
+    for i, (rows, cols) in enumerate(((nup, h), (h, u))):
+        q = quantize_int4(torch.randn(e, rows, cols, generator=g) * cols ** -0.5, group, sdt)
+        b = q.packed.view(torch.uint8).int()
+        nib = torch.stack([b & 15, b >> 4], -1).view(e, rows, cols)
+        nib = torch.where(nib > 7, nib - 16, nib).float()
+        vals.append((nib * q.scales.float().repeat_interleave(group, -1)).to(torch.bfloat16).double())
+        pair = act == "swiglu" and i == 0
+        c, s = q.packed, q.scales
+        if pair:
+            c, s = interleave_gate_up(c[:, :u], c[:, u:]), interleave_gate_up(s[:, :u], s[:, u:])
+        codes.append(c.contiguous().to(dev))
+        scales.append(s.contiguous().to(dev))
+        out = torch.empty_like(codes[-1])
+        n8.check(n8.lib().smoe_pack_int4_qtiles(codes[-1].data_ptr(), e, rows, cols, out.data_ptr(),
+                                                n8.stream_of(torch.device(dev))), "pack_int4_qtiles")
+        tiles.append(out)
+    bu, bd = torch.randn(e, u, generator=g) * 0.1, torch.randn(e, h, generator=g) * 0.1
+    bu_d, bd_d = bu.to(dev), bd.to(dev)
+    ex = _experts_struct(n8, n8.INT4, n8.ACT_SWIGLU if act == "swiglu" else n8.ACT_GELU, e, h, u, *codes,
+                         s_up=scales[0], s_down=scales[1], b_up=bu_d, b_down=bd_d, group=group,
+                         scale_dtype=n8.F16 if sdt == torch.float16 else n8.F32)
+    plain = _run_delta(n8, ex, x.to(dev), idx.to(dev), w.to(dev)).double()
+    ex.w_up_tiles, ex.w_down_tiles = tiles[0].data_ptr(), tiles[1].data_ptr()
+    tiled = _run_delta(n8, ex, x.to(dev), idx.to(dev), w.to(dev)).double()
+    ref, bound = torch.zeros(n, h).double(), torch.zeros(n, h).double()
+    for t in range(n):
+        for j in range(k):
+            i = int(idx[t, j])
+            up = x[t].double() @ vals[0][i].t()
+            if act == "swiglu":
+                a = torch.nn.functional.silu(up[:u]) * (up[u:] + bu[i].double())
+            else:
+                a = torch.nn.functional.gelu(up + bu[i].double())
+            r = (a @ vals[1][i].t() + bd[i].double()) * w[t, j].double()
+            mag = (a.abs() @ vals[1][i].abs().t() + bd[i].abs().double()) * w[t, j].double()
+            ref[t] += r
+            # bf16 activations and rows: 2^-9 of each product and of the row
+            bound[t] += (2.0 ** -9 + (2 * u + 2 * h) * 2.0 ** -24 + 1e-5) * mag + 2.0 ** -9 * r.abs() + 1e-6
+    for y in (plain, tiled):
+        assert bool(((y - ref).abs() <= 1.01 * bound).all()), float(((y - ref).abs() / bound).max())

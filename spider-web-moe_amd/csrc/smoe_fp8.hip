@@ -12,10 +12,9 @@ namespace smoe {
 namespace {
 
 typedef int i32x8 __attribute__((ext_vector_type(8)));
-typedef __attribute__((address_space(3))) void* lds_ptr;
-typedef __attribute__((address_space(1))) void* gbl_ptr;
 
 constexpr float kE4m3Max = 448.0f;
+constexpr int kAmaxParts = 1024;  // workgroups (and partials) of the amax pass
 
 // max that keeps a NaN once seen (torch's amax propagates NaN)
 __device__ __forceinline__ float nan_max(float m, float a) { return (a > m || a != a) ? a : m; }
@@ -58,15 +57,50 @@ __device__ __forceinline__ float load_x(const void* x, int64_t i) {
   else return static_cast<float>(reinterpret_cast<const _Float16*>(x)[i]);
 }
 
-// Partial amax |x| of each workgroup's grid-stride share.
+// Whether eight consecutive elements load as 16-byte vectors.
+template <int XDT>
+__device__ __forceinline__ bool vec8(const void* x) {
+  return reinterpret_cast<uintptr_t>(x) % 16 == 0;
+}
+
+// Elements i .. i + 7 (i a multiple of 8, x as vec8 asks).
+template <int XDT>
+__device__ __forceinline__ void load_x8(const void* x, int64_t i, float (&v)[8]) {
+  if constexpr (XDT == SMOE_F32) {
+    const f32x4* p = reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(x) + i);
+    const f32x4 a = p[0], b = p[1];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v[j] = a[j];
+      v[4 + j] = b[j];
+    }
+  } else {
+    const u32x4 a = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(x) + i);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const uint16_t h = static_cast<uint16_t>(a[j >> 1] >> (16 * (j & 1)));
+      v[j] = XDT == SMOE_BF16 ? bf2f(h) : static_cast<float>(__builtin_bit_cast(_Float16, h));
+    }
+  }
+}
+
+// Partial amax |x| of each workgroup's grid-stride share: 8 elements a lane
+// and load, the rest one by one (n % 8, unaligned x).
 template <int XDT>
 __global__ __launch_bounds__(256) void k_amax_partial(const void* __restrict__ x, int64_t n,
                                                       float* __restrict__ partial) {
   __shared__ float red[4];
   float m = 0.f;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < n;
-       i += static_cast<int64_t>(gridDim.x) * 256)
-    m = nan_max(m, fabsf(load_x<XDT>(x, i)));
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
+  const int64_t octs = vec8<XDT>(x) ? n >> 3 : 0;
+  for (int64_t o = t; o < octs; o += stride) {
+    float v[8];
+    load_x8<XDT>(x, 8 * o, v);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) m = nan_max(m, fabsf(v[j]));
+  }
+  for (int64_t i = 8 * octs + t; i < n; i += stride) m = nan_max(m, fabsf(load_x<XDT>(x, i)));
   m = wave_nan_max(m);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
   __syncthreads();
@@ -75,31 +109,55 @@ __global__ __launch_bounds__(256) void k_amax_partial(const void* __restrict__ x
 }
 
 // scale = max(amax / 448, 1e-12) (quant.py:30-33), codes = e4m3(x / scale)
-// (quant.py:52), 4 codes per thread; columns cols .. ld_out-1 of each row
-// are written as code 0 (value 0: the GEMM's K padding).
+// (quant.py:52), 8 codes per thread (4 where rows are not whole 16-byte
+// vectors); columns cols .. ld_out-1 of each row are written as code 0 (value
+// 0: the GEMM's K padding).  Every workgroup reduces the partials itself, its
+// 256 threads loading them at once; one wave in a loop of 16 dependent loads
+// was half the launch (4096 x 1024 bf16: 15.6 -> 9.0 us with the wider
+// accesses, the amax pass 6.3 -> 4.1).
 template <int XDT>
 __global__ __launch_bounds__(256) void k_quant_fp8(const void* __restrict__ x, int rows, int cols,
                                                    int ld_out, const float* __restrict__ partial,
                                                    int nparts, uint8_t* __restrict__ codes,
                                                    float* __restrict__ scale_out) {
-  __shared__ float s_scale;
-  if (threadIdx.x < 64) {
+  __shared__ float red[4];
+  {
+    float v[kAmaxParts / 256];
+#pragma unroll
+    for (int i = 0; i < kAmaxParts / 256; ++i)  // unconditional loads at clamped indices
+      v[i] = partial[min(static_cast<int>(threadIdx.x) + 256 * i, nparts - 1)];
     float m = 0.f;
-    for (int i = threadIdx.x; i < nparts; i += 64) m = nan_max(m, partial[i]);
+#pragma unroll
+    for (int i = 0; i < kAmaxParts / 256; ++i) m = nan_max(m, v[i]);
     m = wave_nan_max(m);
-    if (threadIdx.x == 0) {
-      float sc = __fdiv_rn(m, kE4m3Max);
-      sc = sc < 1e-12f ? 1e-12f : sc;  // clamp_min (a NaN scale stays NaN)
-      s_scale = sc;
-      if (blockIdx.x == 0) *scale_out = sc;
-    }
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
   }
   __syncthreads();
-  const float sc = s_scale;
+  float sc = __fdiv_rn(nan_max(nan_max(red[0], red[1]), nan_max(red[2], red[3])), kE4m3Max);
+  sc = sc < 1e-12f ? 1e-12f : sc;  // clamp_min (a NaN scale stays NaN)
+  if (blockIdx.x == 0 && threadIdx.x == 0) *scale_out = sc;
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
+  if (vec8<XDT>(x) && cols % 8 == 0 && ld_out % 8 == 0 && reinterpret_cast<uintptr_t>(codes) % 8 == 0) {
+    const int octs = ld_out >> 3;
+    const int64_t total = static_cast<int64_t>(rows) * octs;
+    for (int64_t o = t; o < total; o += stride) {
+      const int r = static_cast<int>(o / octs);
+      const int c = static_cast<int>(o - static_cast<int64_t>(r) * octs) * 8;
+      u32x2 w = {0u, 0u};
+      if (c < cols) {
+        float v[8];
+        load_x8<XDT>(x, static_cast<int64_t>(r) * cols + c, v);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) w[j >> 2] |= f32_to_e4m3(__fdiv_rn(v[j], sc)) << (8 * (j & 3));
+      }
+      *reinterpret_cast<u32x2*>(codes + static_cast<int64_t>(r) * ld_out + c) = w;
+    }
+    return;
+  }
   const int quads = ld_out >> 2;
   const int64_t total = static_cast<int64_t>(rows) * quads;
-  for (int64_t q = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; q < total;
-       q += static_cast<int64_t>(gridDim.x) * 256) {
+  for (int64_t q = t; q < total; q += stride) {
     const int r = static_cast<int>(q / quads);
     const int c0 = static_cast<int>(q - static_cast<int64_t>(r) * quads) * 4;
     uint32_t word = 0;
@@ -144,99 +202,62 @@ __global__ __launch_bounds__(256) void k_quant_fp8_rows(const void* __restrict__
   }
 }
 
-// LDS rows of 64 B, chunk c of row r at c ^ ((r >> 1) & 3) (the ring
-// kernels' conflict-free layout).
-__device__ __forceinline__ int swz64(int row, int chunk) {
-  return row * 64 + ((chunk ^ ((row >> 1) & 3)) << 4);
-}
-
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (0xF << 8));
-}
-__device__ __forceinline__ void wait_lgkm() { __builtin_amdgcn_s_waitcnt(0xC07F); }
-
 // out[m, n] = act(xs * ws * sum_k X[m, k] W[n, k] + bias[n]) over e4m3
 // codes X [N, ldx], W [N_out, ldw] (K a multiple of 256, zero-padded).
 //
 // 128 x 128 block tile, 4 waves in a 2 x 2 grid (wave tile 64 x 64), K
-// advancing 128 per stage through a 3-stage LDS ring (32 KB a stage) fed
-// by global_load_lds_dwordx4.  A stage keeps each operand as two 64-byte
-// halves of its 128-byte k slice ([X k 0-63][X k 64-127][W k 0-63][W k
-// 64-127], 8 KB each, the swizzle above); a lane's 32-byte MFMA fragment
-// (row l % 16, k bytes 32 (l / 16) ..) is two ds_read_b128 from one half.
-// Both operands use the same lane -> k assignment, so every lane group
-// multiplies matching k.  Fragments of stage s+1 are read into a second
-// register set while stage s's 16 MFMAs run.
+// advancing 128 per stage (128-byte rows, swizzled as sw_chunk says) through a
+// 2-stage LDS ring (32 KB a stage) fed by global_load_lds_dwordx4; a lane's
+// 32-byte MFMA fragment (row l % 16, k bytes 32 (l / 16) ..) is two
+// ds_read_b128.  Both operands use the same lane -> k assignment, so every lane
+// group multiplies matching k.  A launch is a few stages long (K 1024: 8) and
+// waits for memory in every one, so two workgroups share a CU.  1024 -> 2816,
+// 4096 rows, bf16 out: 44.5 -> 27 us (875 TFLOP/s) against one workgroup with
+// a 3-stage ring of 64-byte rows, fragments a stage ahead in registers and
+// 8-byte stores.  Workgroup ids are dealt to the 8 XCDs round robin and each
+// XCD takes one contiguous part of the tiles, row tile by row tile, so its
+// rows and the weights stay in its L2.
 template <int EPI, int ODT>
-__global__ __launch_bounds__(256) void k_gemm_f8f8(const uint8_t* __restrict__ X, int ldx,
-                                                   const uint8_t* __restrict__ W, int ldw,
-                                                   const float* __restrict__ xs,
-                                                   const float* __restrict__ ws,
-                                                   const float* __restrict__ bias, int N, int K,
-                                                   int N_out, void* __restrict__ out, int ldo,
-                                                   int tiles_m) {
-  constexpr int BM = 128, BN = 128, NS = 3, SUB = 128 * 64, STAGE = 4 * SUB, LD = 8;
+__global__ __launch_bounds__(256, 2) void k_gemm_f8f8(const uint8_t* __restrict__ X, int ldx,
+                                                      const uint8_t* __restrict__ W, int ldw,
+                                                      const float* __restrict__ xs,
+                                                      const float* __restrict__ ws,
+                                                      const float* __restrict__ bias, int N, int K,
+                                                      int N_out, void* __restrict__ out, int ldo,
+                                                      int tiles_n) {
+  constexpr int BM = 128, BN = 128, NS = 2, OPB = 128 * 128, STAGE = 2 * OPB, LD = 8;
   __shared__ __attribute__((aligned(1024))) uint8_t ring[NS * STAGE];
-  const int tm = blockIdx.x % tiles_m, tn = blockIdx.x / tiles_m;
-  const int m0 = tm * BM, n0 = tn * BN;
+  const int T = gridDim.x, x = blockIdx.x & 7, rem = T & 7;
+  const int logical = x * (T >> 3) + min(x, rem) + (blockIdx.x >> 3);
+  const int m0 = logical / tiles_n * BM, n0 = logical % tiles_n * BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
 
-  // DMA: instruction q = wave + 4 j (j < 8) of a stage covers operand q >> 4
-  // (0 X, 1 W), half (q >> 3) & 1, rows 16 (q & 7) ..; lane i: row i / 4,
-  // physical chunk i % 4, loading the logical chunk the swizzle puts there
+  // DMA: instruction j of this wave covers rows 8 (4 (j % 4) + wave) .. of
+  // operand j / 4 (X, W); lane i: row i / 8, physical chunk i % 8, loading the
+  // logical chunk the swizzle puts there
   const uint8_t* src[LD];
-  int dst[LD];
-  {
-    const int pr = lane >> 2, pc = lane & 3;
 #pragma unroll
-    for (int j = 0; j < LD; ++j) {
-      const int q = wave + 4 * j;
-      const int op = q >> 4, half = (q >> 3) & 1, rb = q & 7;
-      const int r = rb * 16 + pr;
-      const int lc = pc ^ ((r >> 1) & 3);
-      if (op == 0) {
-        const int row = m0 + r < N ? m0 + r : N - 1;  // rows past the end: valid data, never stored
-        src[j] = X + static_cast<int64_t>(row) * ldx + 64 * half + 16 * lc;
-      } else {
-        const int row = n0 + r < N_out ? n0 + r : N_out - 1;
-        src[j] = W + static_cast<int64_t>(row) * ldw + 64 * half + 16 * lc;
-      }
-      dst[j] = (op * 2 + half) * SUB + rb * 1024;
-    }
+  for (int j = 0; j < LD; ++j) {
+    const int r = 8 * (4 * (j & 3) + wave) + (lane >> 3), c = 16 * sw_chunk<8>(r, lane & 7);
+    // rows past the end: valid data, never stored
+    src[j] = j < 4 ? X + static_cast<int64_t>(min(m0 + r, N - 1)) * ldx + c
+                   : W + static_cast<int64_t>(min(n0 + r, N_out - 1)) * ldw + c;
   }
   auto issue = [&](int stage) {
     uint8_t* base = ring + (stage % NS) * STAGE;
-    const int k0 = stage * 128;
 #pragma unroll
     for (int j = 0; j < LD; ++j)
-      __builtin_amdgcn_global_load_lds((gbl_ptr)(src[j] + k0), (lds_ptr)(base + dst[j]), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((gbl_vptr)(src[j] + static_cast<int64_t>(stage) * 128),
+                                       (lds_vptr)(base + (j >> 2) * OPB + (4 * (j & 3) + wave) * 1024),
+                                       16, 0, 0);
   };
-
   const int fr = lane & 15, g = lane >> 4;
-  const int half = g >> 1, c0 = 2 * (g & 1);
-  i32x8 xa[4], wa[4], xb[4], wb[4];
-  auto read_frags = [&](int stage, i32x8 (&xf)[4], i32x8 (&wf)[4]) {
-    const uint8_t* sx = ring + (stage % NS) * STAGE + half * SUB;
-    const uint8_t* sw = sx + 2 * SUB;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = wm * 64 + i * 16 + fr;
-      const u32x4 lo = *reinterpret_cast<const u32x4*>(sx + swz64(r, c0));
-      const u32x4 hi = *reinterpret_cast<const u32x4*>(sx + swz64(r, c0 + 1));
-      xf[i] = __builtin_bit_cast(i32x8, (uint32_t __attribute__((ext_vector_type(8)))){
-                                            lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w});
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int r = wn * 64 + j * 16 + fr;
-      const u32x4 lo = *reinterpret_cast<const u32x4*>(sw + swz64(r, c0));
-      const u32x4 hi = *reinterpret_cast<const u32x4*>(sw + swz64(r, c0 + 1));
-      wf[j] = __builtin_bit_cast(i32x8, (uint32_t __attribute__((ext_vector_type(8)))){
-                                            lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w});
-    }
+  auto frag = [&](const uint8_t* op, int r) {
+    const u32x4 lo = *reinterpret_cast<const u32x4*>(op + r * 128 + (sw_chunk<8>(r, 2 * g) << 4));
+    const u32x4 hi = *reinterpret_cast<const u32x4*>(op + r * 128 + (sw_chunk<8>(r, 2 * g + 1) << 4));
+    return __builtin_bit_cast(i32x8, (uint32_t __attribute__((ext_vector_type(8)))){
+                                         lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w});
   };
 
   f32x4 acc[4][4];
@@ -245,54 +266,76 @@ __global__ __launch_bounds__(256) void k_gemm_f8f8(const uint8_t* __restrict__ X
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const int KT = K / 128;  // even: K % 256 == 0
-  auto step = [&](int s, i32x8 (&xc)[4], i32x8 (&wc)[4], i32x8 (&xn)[4], i32x8 (&wn_)[4]) {
-    if (s + 1 < KT) {
-      if (s + NS - 1 < KT) wait_vm<(NS - 2) * LD>();
-      else wait_vm<0>();
-      wait_lgkm();
-      __builtin_amdgcn_s_barrier();
-      if (s + NS < KT) issue(s + NS);  // into stage s's slot: its fragments are in registers
-      read_frags(s + 1, xn, wn_);
-    }
+  const int KT = K / 128;
+  issue(0);
+  for (int s = 0; s < KT; ++s) {
+    // own part of stage s landed; after the barrier everybody's, and nobody
+    // reads stage s - 1 any more
+    wait_vmcnt<0>();
+    wait_lgkm0();
+    __builtin_amdgcn_s_barrier();
+    if (s + 1 < KT) issue(s + 1);  // into the slot of stage s - 1
+    const uint8_t* sx = ring + (s % NS) * STAGE;
+    i32x8 xf[4], wf[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) xf[i] = frag(sx, wm * 64 + i * 16 + fr);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) wf[j] = frag(sx + OPB, wn * 64 + j * 16 + fr);
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        acc[j][i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wc[j], xc[i], acc[j][i], 0, 0, 0,
+        acc[j][i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[j], xf[i], acc[j][i], 0, 0, 0,
                                                                      0, 0, 0);
-  };
-
-#pragma unroll
-  for (int st = 0; st < NS; ++st)
-    if (st < KT) issue(st);
-  if (KT >= NS) wait_vm<(NS - 1) * LD>();
-  else wait_vm<0>();
-  __builtin_amdgcn_s_barrier();
-  read_frags(0, xa, wa);
-  for (int s = 0; s < KT; s += 2) {
-    step(s, xa, wa, xb, wb);
-    step(s + 1, xb, wb, xa, wa);
   }
 
   // epilogue: lane holds channels n .. n+3 (4 (l / 16) + v) of row m (l % 16)
   const float sc = xs[0] * ws[0];
+  float b4[4][4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int n = n0 + wn * 64 + j * 16 + 4 * g;
-    float b4[4];
 #pragma unroll
-    for (int v = 0; v < 4; ++v) b4[v] = (bias && n + v < N_out) ? bias[n + v] : 0.f;
+    for (int v = 0; v < 4; ++v) b4[j][v] = (bias && n + v < N_out) ? bias[n + v] : 0.f;
+  }
+  auto value = [&](int i, int j, int v) {
+    const float y = acc[j][i][v] * sc + b4[j][v];
+    return EPI == 1 ? gelu_erf(y) : y;
+  };
+  if constexpr (ODT == SMOE_BF16) {
+    // whole 16-byte chunks: the tile is staged in the ring (chunk c of row r
+    // at c ^ (r & 15)) and leaves in rows of 256 bytes
+    if (N_out % 8 == 0 && ldo % 8 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0) {
+      uint16_t* stg = reinterpret_cast<uint16_t*>(ring);
+      auto at = [&](int r, int c) { return stg + r * BN + ((((c >> 3) ^ (r & 15)) << 3) | (c & 7)); };
+      __syncthreads();  // every wave is done with the ring
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          *reinterpret_cast<u32x2*>(at(wm * 64 + i * 16 + fr, wn * 64 + j * 16 + 4 * g)) =
+              u32x2{pack_bf2(value(i, j, 0), value(i, j, 1)), pack_bf2(value(i, j, 2), value(i, j, 3))};
+      __syncthreads();
+      for (int q = tid; q < BM * (BN / 8); q += 256) {
+        const int r = q / (BN / 8), c = q % (BN / 8) * 8;
+        if (m0 + r < N && n0 + c < N_out)
+          *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(out) +
+                                    static_cast<int64_t>(m0 + r) * ldo + n0 + c) =
+              *reinterpret_cast<const u32x4*>(at(r, c));
+      }
+      return;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int n = n0 + wn * 64 + j * 16 + 4 * g;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int m = m0 + wm * 64 + i * 16 + fr;
       if (m >= N) continue;
       float o[4];
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const float y = acc[j][i][v] * sc + b4[v];
-        o[v] = EPI == 1 ? gelu_erf(y) : y;
-      }
+      for (int v = 0; v < 4; ++v) o[v] = value(i, j, v);
       const int64_t base = static_cast<int64_t>(m) * ldo + n;
       if (ODT == SMOE_F32) {
         float* po = reinterpret_cast<float*>(out) + base;
@@ -319,8 +362,6 @@ __global__ __launch_bounds__(256) void k_gemm_f8f8(const uint8_t* __restrict__ X
 
 int rc() { return hipGetLastError() == hipSuccess ? SMOE_OK : SMOE_EHIP; }
 
-constexpr int kAmaxParts = 1024;
-
 }  // namespace
 
 size_t quantize_fp8_workspace_bytes() { return kAmaxParts * sizeof(float); }
@@ -345,7 +386,7 @@ int launch_quantize_fp8(const void* x, int xdt, int rows, int cols, int ld_out, 
   const int parts = static_cast<int>(std::min<int64_t>(kAmaxParts, (n + 4095) / 4096));
   float* partial = static_cast<float*>(workspace);
   const int64_t quads = static_cast<int64_t>(rows) * (ld_out / 4);
-  const int qblocks = static_cast<int>(std::min<int64_t>(4096, (quads + 255) / 256));
+  const int qblocks = static_cast<int>(std::min<int64_t>(2048, (quads + 511) / 512));
   auto run = [&](auto xd) {
     constexpr int XD = decltype(xd)::value;
     hipLaunchKernelGGL((k_amax_partial<XD>), dim3(parts), dim3(256), 0, s, x, n, partial);
@@ -369,10 +410,11 @@ int launch_gemm_f8f8(const uint8_t* xq, int ldx, const float* xs, const uint8_t*
     return SMOE_EINVAL;
   if (N == 0) return SMOE_OK;
   const int tiles_m = (N + 127) / 128, tiles_n = (N_out + 127) / 128;
+  if (static_cast<int64_t>(tiles_m) * tiles_n > 0x7fffffff) return SMOE_EINVAL;
   const dim3 grid(tiles_m * tiles_n), block(256);
   auto go = [&](auto epi, auto od) {
     SMOE_LAUNCH((k_gemm_f8f8<decltype(epi)::value, decltype(od)::value>), grid, block, 0, s, xq,
-                ldx, wq, ldw, xs, ws, bias, N, K, N_out, out, ldo, tiles_m);
+                ldx, wq, ldw, xs, ws, bias, N, K, N_out, out, ldo, tiles_n);
     return rc();
   };
   using I0 = std::integral_constant<int, 0>;

@@ -1048,8 +1048,8 @@ SMOE_API int smoe_dispatch_plan(const int32_t* idx, const float* w, int N, int K
   float* tw = at<float>(ws, z.take(static_cast<size_t>(N) * K * 4));
   int32_t* acnt = at<int32_t>(ws, z.take(E * 4));
   void* scratch = at<void>(ws, z.take(plan_scratch_bytes(N, E)));
-  SMOE_TRY(launch_merge_slots(idx, w, N, K, E, 1, tg, tw, s), "merge slots");
-  SMOE_TRY(launch_plan(tg, tw, N, K, E, 1, counts, acnt, offsets, rows, row_w, tok_row, scratch, s),
+  SMOE_TRY(launch_merge_plan(idx, w, N, K, E, tg, tw, counts, acnt, offsets, rows, row_w, tok_row,
+                             scratch, s),
            "plan");
   return SMOE_OK;
 }

@@ -156,15 +156,8 @@ int launch_route_topk(const float* logits, int N, int E, int K, int32_t* top_idx
 // an expert and are dropped, as in the reference; drop_nonpos also drops
 // merged weights <= 0 (sparse_experts.py:56).  w == nullptr: every slot
 // weighs 1 (a binary source mask, model.py:277-279).
-__global__ __launch_bounds__(256) void k_merge_slots(const int32_t* __restrict__ idx,
-                                                     const float* __restrict__ w, int N, int K,
-                                                     int E, int drop_nonpos,
-                                                     int32_t* __restrict__ tok_g,
-                                                     float* __restrict__ tok_w) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= N) return;
-  const int32_t* ti = idx + static_cast<int64_t>(t) * K;
-  const float* tw = w ? w + static_cast<int64_t>(t) * K : nullptr;
+__device__ __forceinline__ void merge_token(const int32_t* ti, const float* tw, int K, int E,
+                                            int drop_nonpos, int32_t* og, float* ow) {
   int out = 0;
   int last = -1;
   // emit groups in ascending order: repeatedly take the smallest id > last
@@ -180,14 +173,25 @@ __global__ __launch_bounds__(256) void k_merge_slots(const int32_t* __restrict__
       if (ti[s] == best) acc = acc + (tw ? tw[s] : 1.f);
     last = best;
     if (drop_nonpos && !(acc > 0.f)) continue;
-    tok_g[static_cast<int64_t>(t) * K + out] = best;
-    tok_w[static_cast<int64_t>(t) * K + out] = acc;
+    og[out] = best;
+    ow[out] = acc;
     ++out;
   }
   for (; out < K; ++out) {
-    tok_g[static_cast<int64_t>(t) * K + out] = -1;
-    tok_w[static_cast<int64_t>(t) * K + out] = 0.f;
+    og[out] = -1;
+    ow[out] = 0.f;
   }
+}
+
+__global__ __launch_bounds__(256) void k_merge_slots(const int32_t* __restrict__ idx,
+                                                     const float* __restrict__ w, int N, int K,
+                                                     int E, int drop_nonpos,
+                                                     int32_t* __restrict__ tok_g,
+                                                     float* __restrict__ tok_w) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= N) return;
+  const int64_t e0 = static_cast<int64_t>(t) * K;
+  merge_token(idx + e0, w ? w + e0 : nullptr, K, E, drop_nonpos, tok_g + e0, tok_w + e0);
 }
 
 int launch_merge_slots(const int32_t* idx, const float* w, int N, int K, int E, int drop_nonpos,
@@ -837,6 +841,40 @@ int launch_plan(const int32_t* tok_g, const float* tok_w, int N, int S, int G, i
   return hipGetLastError() == hipSuccess ? SMOE_OK : SMOE_EHIP;
 }
 
+// Slot merge and chunk ranks in one launch, a workgroup per 64-token chunk:
+// the chunk's slots go through LDS (merged by one thread per token), and the
+// four waves rank its groups in W windows (K <= kMergeRankMaxK).
+constexpr int kMergeRankMaxK = 16;
+
+__global__ __launch_bounds__(256) void k_merge_rank(const int32_t* __restrict__ idx,
+                                                    const float* __restrict__ w, int N, int K,
+                                                    int G, int drop, int C, int W,
+                                                    int32_t* __restrict__ tok_g,
+                                                    float* __restrict__ tok_w,
+                                                    int32_t* __restrict__ ccnt,
+                                                    int32_t* __restrict__ cacnt,
+                                                    int32_t* __restrict__ tokrow) {
+  __shared__ int32_t in_g[64 * kMergeRankMaxK], sg[64 * kMergeRankMaxK];
+  __shared__ float in_w[64 * kMergeRankMaxK], sw[64 * kMergeRankMaxK];
+  const int chunk = blockIdx.x, t0 = chunk * 64, tid = threadIdx.x;
+  const int n = min(64, N - t0), m = n * K;
+  const int64_t e0 = static_cast<int64_t>(t0) * K;
+  for (int i = tid; i < m; i += 256) {
+    in_g[i] = idx[e0 + i];
+    in_w[i] = w[e0 + i];
+  }
+  __syncthreads();
+  if (tid < n) merge_token(in_g + tid * K, in_w + tid * K, K, G, drop, sg + tid * K, sw + tid * K);
+  __syncthreads();
+  for (int i = tid; i < m; i += 256) {
+    tok_g[e0 + i] = sg[i];
+    tok_w[e0 + i] = sw[i];
+  }
+  const int win = (G + W - 1) / W;
+  for (int i = tid >> 6; i * win < G; i += 4)
+    rank_chunk(sg, sw, N, K, G, drop, t0, i * win, win, ccnt + chunk, cacnt + chunk, C, tokrow, t0);
+}
+
 // The scan and scatter of two plans (the expert plan and the destination
 // plan of one loop) whose chunk ranks are in place, one launch each: each
 // launch's workgroups are split between the plans, which use the same device
@@ -942,6 +980,33 @@ __global__ __launch_bounds__(256) void k_plan2_finish(const Plan2 a, const Plan2
   __syncthreads();
   block_group_offsets(tot, p.G, goff, wsum);
   scatter_block(p, blk, N, base, C, goff);
+}
+
+int launch_merge_plan(const int32_t* idx, const float* w, int N, int K, int G, int32_t* tok_g,
+                      float* tok_w, int32_t* cnt, int32_t* acnt, int32_t* off, int32_t* rows,
+                      float* roww, int32_t* tokrow, void* scratch, hipStream_t s) {
+  if (G < 1 || G > kPlanMaxG || K < 1 || K > kPlanMaxS || N < 0) return SMOE_EINVAL;
+  const int C = (N + 63) / 64;
+  if (N <= 64 || K > kMergeRankMaxK) {
+    const int rc = launch_merge_slots(idx, w, N, K, G, 1, tok_g, tok_w, s);
+    return rc != SMOE_OK ? rc : launch_plan(tok_g, tok_w, N, K, G, 1, cnt, acnt, off, rows, roww,
+                                            tokrow, scratch, s);
+  }
+  const int W = max(4, (G + 63) / 64);  // a window per wave
+  int32_t* ccnt = reinterpret_cast<int32_t*>(scratch);
+  int32_t* cacnt = ccnt + static_cast<int64_t>(C) * G;
+  hipLaunchKernelGGL(k_merge_rank, dim3(C), dim3(256), 0, s, idx, w, N, K, G, 1, C, W, tok_g, tok_w,
+                     ccnt, cacnt, tokrow);
+  if (C <= kFinishMaxC && G <= kFinishMaxG) {
+    Plan2 a{tok_g, tok_w, K, G, 1, cnt, acnt, off, rows, roww, tokrow, ccnt, cacnt,
+            nullptr, nullptr, nullptr, nullptr, 0};
+    hipLaunchKernelGGL(k_plan2_finish, dim3((N + 255) / 256), dim3(256), 0, s, a, a, N, C);
+  } else {
+    hipLaunchKernelGGL(k_plan_scan, dim3(G), dim3(64), 0, s, C, ccnt, cacnt, cnt, acnt);
+    hipLaunchKernelGGL(k_plan_scatter, dim3((N + 255) / 256), dim3(256), 0, s, tok_g, tok_w, N, K,
+                       G, C, ccnt, cnt, off, rows, roww, tokrow);
+  }
+  return hipGetLastError() == hipSuccess ? SMOE_OK : SMOE_EHIP;
 }
 
 int launch_plan2_finish(const PlanSpec& pa, const PlanSpec& pb, int N, void* scratch,

@@ -61,9 +61,11 @@ __device__ __forceinline__ bool mid_tile(const GemmArgs& p, int bid, int& g, int
 // BM x BN tile, WM x WN waves, K in 64-wide stages that go global -> LDS by
 // DMA (weights in their storage format, widened as the fragments are read)
 // through an NS-stage ring, NS - 1 stages in flight while one computes.  A
-// stage's two MFMAs take its lower and its upper 32 k, so every output is
-// summed in the order of the other large-tile kernels.  LDS rows are swizzled
-// as sw_chunk says.
+// stage's two MFMAs take its lower and its upper 32 k, the order of the other
+// large-tile kernels, or with PAIRS the low and the high 8 of the 16 k at
+// 16 q of lane quarter q, the order of k_gemm_stream4 (fp8: one 16-byte
+// fragment read then holds both).  LDS rows are swizzled as sw_chunk
+// says.
 //
 // Bound: the operand stream into the CUs and its latency (with the MFMAs and
 // fragment reads taken out a launch keeps 85-95% of its time; fragments read
@@ -73,7 +75,7 @@ __device__ __forceinline__ bool mid_tile(const GemmArgs& p, int bid, int& g, int
 // small rings and two or three workgroups per CU beat one deep ring (H 1024
 // -> 2816 GELU, 16 groups of 250 rows: 128 x 128 tiles, 2 stages, 2
 // workgroups per CU 51 us; 4 stages, 8 waves, 1 per CU 71 us).
-template <int FMT, int EPI, int BM, int BN, int WM, int WN, int NS, int OCC>
+template <int FMT, int EPI, int BM, int BN, int WM, int WN, int NS, int OCC, bool PAIRS>
 __global__ __launch_bounds__(WM* WN * 64, OCC) void k_gemm_mid(const GemmArgs p) {
   constexpr int NW = WM * WN, TM = BM / WM, TN = BN / WN, FM = TM / 16, FN = TN / 16;
   constexpr int WB = mid_wb<FMT>(), CPR = WB / 16;
@@ -84,6 +86,7 @@ __global__ __launch_bounds__(WM* WN * 64, OCC) void k_gemm_mid(const GemmArgs p)
   static_assert(A_LD * NW * 1024 == A_BYTES && W_LD * NW * 1024 == BN * WB, "whole DMA instructions");
   static_assert(EPI != EPI_SWIGLU || TN % 64 == 0, "SwiGLU pairs channel c with c + 32");
   static_assert(NS * STAGE >= BM * BN * 2, "the output tile is staged in the ring");
+  static_assert(!PAIRS || FMT != SMOE_INT4, "int4 at these row counts: k_gemm_stream4");
   __shared__ __attribute__((aligned(1024))) uint8_t ring[NS * STAGE + SCALES];
   int g, m0, mrows, n0;
   if (!mid_tile<BM, BN>(p, blockIdx.x, g, m0, mrows, n0)) return;  // uniform
@@ -142,6 +145,7 @@ __global__ __launch_bounds__(WM* WN * 64, OCC) void k_gemm_mid(const GemmArgs p)
   for (int st = 0; st < NS - 1; ++st)
     if (st < KC) issue(st);
   const bool live = wm * TM < mrows;  // this wave has rows
+  auto k8 = [&](int h) { return PAIRS ? 2 * q + h : 4 * h + q; };  // the 8 k of MFMA h, in eights
   for (int kc = 0; kc < KC; ++kc) {
     // own part of stage kc landed (later ones may fly); after the barrier
     // everybody's, and nobody reads stage kc - 1 any more
@@ -160,14 +164,18 @@ __global__ __launch_bounds__(WM* WN * 64, OCC) void k_gemm_mid(const GemmArgs p)
       const uint8_t* wr = sw + row * WB;
       float scale = 0.f;
       if constexpr (FMT == SMOE_INT4) scale = stab[((kc * 64) >> gs_shift) * BN + row];
+      u32x4 both = {0u, 0u, 0u, 0u};
+      if constexpr (FMT == SMOE_FP8_E4M3 && PAIRS)
+        both = *reinterpret_cast<const u32x4*>(wr + (sw_chunk<CPR>(row, q) << 4));
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         u32x4 v;
         if constexpr (FMT == SMOE_BF16) {
-          v = *reinterpret_cast<const u32x4*>(wr + (sw_chunk<CPR>(row, 4 * h + q) << 4));
+          v = *reinterpret_cast<const u32x4*>(wr + (sw_chunk<CPR>(row, k8(h)) << 4));
         } else if constexpr (FMT == SMOE_FP8_E4M3) {
-          const u32x2 r = *reinterpret_cast<const u32x2*>(
-              wr + (sw_chunk<CPR>(row, 2 * h + (q >> 1)) << 4) + 8 * (q & 1));
+          u32x2 r;
+          if constexpr (PAIRS) r = u32x2{both[2 * h], both[2 * h + 1]};
+          else r = *reinterpret_cast<const u32x2*>(wr + (sw_chunk<CPR>(row, k8(h) >> 1) << 4) + 8 * (q & 1));
           const u32x2 lo = fp8x4_to_bf16x4(r.x), hi = fp8x4_to_bf16x4(r.y);
           v = u32x4{lo.x, lo.y, hi.x, hi.y};
         } else {
@@ -183,7 +191,7 @@ __global__ __launch_bounds__(WM* WN * 64, OCC) void k_gemm_mid(const GemmArgs p)
       bf16x8 af[2];
 #pragma unroll
       for (int h = 0; h < 2; ++h)
-        af[h] = *reinterpret_cast<const bf16x8*>(sa + r * 128 + (sw_chunk<8>(r, 4 * h + q) << 4));
+        af[h] = *reinterpret_cast<const bf16x8*>(sa + r * 128 + (sw_chunk<8>(r, k8(h)) << 4));
 #pragma unroll
       for (int t = 0; t < FN; ++t)
 #pragma unroll
@@ -212,14 +220,29 @@ __global__ __launch_bounds__(WM* WN * 64, OCC) void k_gemm_mid(const GemmArgs p)
   }
 }
 
+// The order of the sums, by rows per group: up to 128 that of k_gemm_stream4,
+// which keeps the int4 groups of that size, so that the formats agree and a
+// model's results at these sizes are those it has given before; past it that
+// of the general and the prefill tiles, for the same reason.  Neither is
+// faster.
+bool k_pairs(const GemmArgs& a) {
+  return a.G > 0 && a.max_rows / a.G <= 128 && a.fmt != SMOE_INT4;
+}
+
 template <int FMT, int EPI, int BM, int BN, int WM, int WN, int NS, int OCC>
 int launch_tiles(const GemmArgs& a, hipStream_t s) {
   const int64_t rows = a.G == 0 ? a.single_rows : a.max_rows;
   const int64_t wgs = ((rows + BM - 1) / BM + a.G) * ((a.N_out + BN - 1) / BN);
   if (wgs > 0x7fffffff) return SMOE_EINVAL;
   if (wgs == 0) return SMOE_OK;
-  SMOE_LAUNCH((k_gemm_mid<FMT, EPI, BM, BN, WM, WN, NS, OCC>), dim3(static_cast<unsigned>(wgs)),
-              dim3(WM * WN * 64), 0, s, a);
+  const dim3 grid(static_cast<unsigned>(wgs)), block(WM * WN * 64);
+  if constexpr (FMT != SMOE_INT4) {
+    if (k_pairs(a)) {
+      SMOE_LAUNCH((k_gemm_mid<FMT, EPI, BM, BN, WM, WN, NS, OCC, true>), grid, block, 0, s, a);
+      return hipGetLastError() == hipSuccess ? SMOE_OK : SMOE_EHIP;
+    }
+  }
+  SMOE_LAUNCH((k_gemm_mid<FMT, EPI, BM, BN, WM, WN, NS, OCC, false>), grid, block, 0, s, a);
   return hipGetLastError() == hipSuccess ? SMOE_OK : SMOE_EHIP;
 }
 

@@ -275,3 +275,69 @@ def test_fp8fp8_tile_edges(n, k, n_out, act):
 def test_merged_plan_edges(n, k, e):
     import test_gpu_kernels
     test_gpu_kernels.test_dispatch_plan_bit_exact(n, k, e)
+
+
+def _whole_experts(fmt, act, up, down, group=128, tiles=False):
+    """Experts on whole-number weights in -8 .. 7, which every format holds
+    exactly (scales 1): up [e, nup, h] (SwiGLU: gate, then up), down [e, h, u]."""
+    from spider_moe_amd import _native as n8
+    from spider_moe_amd.quant import interleave_gate_up
+    from test_gpu_kernels import _experts_struct
+    e, h, u = down.shape
+    if act == "swiglu":
+        up = interleave_gate_up(up[:, :u], up[:, u:])
+    keep, kw = [], {}
+    for name, m in (("up", up), ("down", down)):
+        if fmt == "bf16":
+            keep.append(m.to(torch.bfloat16).contiguous().to(dev))
+        elif fmt == "fp8":
+            keep.append(m.float().to(torch.float8_e4m3fn).view(torch.uint8).contiguous().to(dev))
+            kw["s_" + name] = torch.ones(m.shape[:2], device=dev)
+        else:
+            q = m.int() & 15
+            keep.append((q[..., ::2] | q[..., 1::2] << 4).to(torch.uint8).contiguous().to(dev))
+            kw["s_" + name] = torch.ones(*m.shape[:2], m.shape[2] // group, dtype=torch.float16, device=dev)
+    if fmt != "bf16":
+        kw["scale_dtype"] = n8.F16 if fmt == "int4" else n8.F32
+    if fmt == "int4":
+        kw["group"] = group
+    code = {"bf16": n8.BF16, "fp8": n8.FP8_E4M3, "int4": n8.INT4}[fmt]
+    ex = _experts_struct(n8, code, n8.ACT_SWIGLU if act == "swiglu" else n8.ACT_GELU, e, h, u, *keep, **kw)
+    if tiles:  # int4
+        for name, m, w in (("up", up, keep[0]), ("down", down, keep[1])):
+            t = torch.empty_like(w)
+            n8.check(n8.lib().smoe_pack_int4_qtiles(w.data_ptr(), e, m.shape[1], m.shape[2], t.data_ptr(),
+                                                    n8.stream_of(torch.device(dev))), "pack_int4_qtiles")
+            setattr(ex, f"w_{name}_tiles", t.data_ptr())
+            keep.append(t)
+    return ex, (keep, kw)
+
+
+def _whole_weights(g, e, h, u, act):
+    nup = 2 * u if act == "swiglu" else u
+    return (torch.randint(-8, 8, (e, nup, h), generator=g), torch.randint(-8, 8, (e, h, u), generator=g))
+
+
+# 33-128 rows per group: every format sums a 64-k step in the order of the
+# int4 stream kernel (MFMAs over the low and the high 8 of 16 consecutive k),
+# so weights that all three hold exactly give the same bits.  36, 97 and 128
+# rows per group on average, 0 to 300 in one; 11 and 2 steps of K
+@pytest.mark.parametrize("n,h,u", [(288, 256, 704), (776, 128, 1408), (1024, 640, 256)])
+@pytest.mark.parametrize("act", ["gelu", "swiglu"])
+def test_grouped_mid_rows_sum_order(n, h, u, act):
+    from spider_moe_amd import _native as n8
+    from test_gpu_kernels import _run_delta
+    say("mid rows, sum order", n, h, u, act)
+    g = torch.Generator().manual_seed(n + u)
+    e, group = 8, 64 if u % 128 else 128
+    ids = torch.multinomial(torch.tensor([.3, .25, .15, .1, .1, .06, .04, 0.]), n, True, generator=g)
+    up, down = _whole_weights(g, e, h, u, act)
+    x = (torch.randn(n, h, generator=g) * 0.05).to(torch.bfloat16)
+    w = torch.rand(n, 1, generator=g) + 0.1
+    got = []
+    for fmt in ("int4", "bf16", "fp8"):
+        ex, keep = _whole_experts(fmt, act, up, down, group)
+        got.append(_run_delta(n8, ex, x.to(dev), ids.int().view(n, 1).to(dev), w.to(dev)))
+    assert bool(got[0].isfinite().all()) and float(got[0].abs().max()) > 0
+    for y in got[1:]:
+        assert torch.equal(y, got[0]), float((y != got[0]).float().mean())

@@ -99,8 +99,8 @@ typedef struct smoe_experts {
    * results for bf16).  int4 (smoe_pack_int4_qtiles): the int4 tile layout,
    * read by the ping-pong GEMM at prefill sizes (>= 256 rows per expert) in
    * place of the general int4 kernel, and by the decode weight stream for
-   * group sizes that are powers of two from 64; the kernels between them keep
-   * reading the packed int4. */
+   * group sizes that are powers of two from 64 (bit-identical results); the
+   * kernels between them keep reading the packed int4. */
   const void* w_up_tiles;
   const void* w_down_tiles;
 } smoe_experts;

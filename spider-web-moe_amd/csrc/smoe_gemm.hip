@@ -829,11 +829,12 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_skinny(const GemmArgs p) {
 // waves of the grid would do their arithmetic at the end).  The KSPLIT waves
 // of a slice add their partial sums through LDS in wave order (bit-identical
 // run to run); with KSPLIT 1 no wave waits for another.  k order inside a
-// 64-wide step, the same for both operands: bf16 weights and int4 tiles take
-// k 8q..8q+7 (first MFMA) and 32+8q.. (second), so each of a bf16 step's two
-// 16-byte loads covers 64 contiguous bytes of 16 rows; fp8 and row-major int4
-// take the 16 consecutive k at 16q.  Only the last 2D - 1 steps' refills sit under a branch, so the
-// main loop's waits count the loads in flight exactly.
+// 64-wide step, the same for both operands: bf16 weights take k 8q..8q+7
+// (first MFMA) and 32+8q.. (second), so each of their two 16-byte loads
+// covers 64 contiguous bytes of 16 rows; fp8 and int4 take the 16
+// consecutive k at 16q, whichever layout they come from.  Only the last
+// 2D - 1 steps' refills sit under a branch, so the main loop's waits count
+// the loads in flight exactly.
 //
 // int4: a scale converted (or its type chosen) where it is loaded waits for
 // that load, and with it for every load before it, so the ring holds the bits
@@ -842,7 +843,8 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_skinny(const GemmArgs p) {
 // contiguous.  64 experts, 16 tokens top-2 (36 MB of codes), us per launch:
 // up 2048 -> 1408 33.5 -> 31.5 (bits) -> 23.9 (tiles), down 32.8 -> 22.3 -> 18.2
 // (2 TB/s; the lookup and the first loads' round trips are half of that; a
-// ring of 6 steps 26.3 and 19.0).
+// ring of 6 steps 26.3 and 19.0).  The lane swaps that keep the row-major sums'
+// order on the tiles cost 3 us of the four loops' 631.
 template <int FMT>
 struct DRaw;
 template <> struct DRaw<SMOE_BF16> { u32x4 a, b; };
@@ -862,6 +864,15 @@ __device__ __forceinline__ int nth_set_bit(uint64_t m, int j) {
     pos += up ? w : 0;
   }
   return pos;
+}
+
+// gfx950's lane swaps: rows of 16 lanes 2, 3 of c.x with rows 0, 1 of c.y; rows
+// 1, 3 of c.x with rows 0, 2 of c.y.
+__device__ __forceinline__ u32x2 swap32(u32x2 c) {
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(c.x, c.y, false, false));
+}
+__device__ __forceinline__ u32x2 swap16(u32x2 c) {
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(c.x, c.y, false, false));
 }
 
 // Whether the first tile of every group has a workgroup row of its own that
@@ -890,7 +901,7 @@ __device__ __forceinline__ void decode_gemm(const GemmArgs& p, int gy, f32x4* re
   static_assert(EPI != EPI_SWIGLU || TNW == 2 || TNW == 4, "SwiGLU slices pair gate and up tiles");
   static_assert(!PK || FMT != SMOE_INT4 || TNW == 4, "an int4 tile block holds 64 channels");
   constexpr bool PK4 = PK && FMT == SMOE_INT4;
-  constexpr bool K32 = FMT == SMOE_BF16 || PK4;  // a step's MFMAs take its lower / upper 32 k
+  constexpr bool K32 = FMT == SMOE_BF16;  // a step's MFMAs take its lower / upper 32 k
   static_assert(!SEL || EPI == EPI_ROWSCALE, "row selection: the edge projection");
   constexpr int BLK = 512 * ESZ2;  // bytes of one 64-k step of a 16-row tile
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1087,8 +1098,16 @@ __device__ __forceinline__ void decode_gemm(const GemmArgs& p, int gy, f32x4* re
         const float sc = SF16 ? static_cast<float>(__builtin_bit_cast(
                                     _Float16, static_cast<uint16_t>(wr[d][t].s)))
                               : __uint_as_float(wr[d][t].s);
-        l = int4x8_to_bf16x8(wr[d][t].a.x, sc);
-        h = int4x8_to_bf16x8(wr[d][t].a.y, sc);
+        u32x2 c = wr[d][t].a;
+        if constexpr (PK4) {
+          // the tile layout gives lane quarter q the 8 k of eights q and 4 + q of
+          // the step; the sums take eights 2q and 2q + 1, so the quarters change
+          // places: (0123, 4567) -> halves (0145, 2367) -> quarters (0246, 1357)
+          c = swap32(c);
+          c = swap16(c);
+        }
+        l = int4x8_to_bf16x8(c.x, sc);
+        h = int4x8_to_bf16x8(c.y, sc);
       }
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {

@@ -341,3 +341,25 @@ def test_grouped_mid_rows_sum_order(n, h, u, act):
     assert bool(got[0].isfinite().all()) and float(got[0].abs().max()) > 0
     for y in got[1:]:
         assert torch.equal(y, got[0]), float((y != got[0]).float().mean())
+
+
+# decode steps on int4 experts: the same bits from the packed rows and from
+# the tile copy (K split over 1, 2 and 4 waves, groups looked up and direct)
+@pytest.mark.parametrize("n,h,u", [(1, 128, 448), (7, 1024, 704), (40, 832, 192), (60, 448, 1408),
+                                   (100, 704, 448)])
+@pytest.mark.parametrize("act", ["gelu", "swiglu"])
+def test_decode_int4_tiles_sum_order(n, h, u, act):
+    from spider_moe_amd import _native as n8
+    from test_gpu_kernels import _run_delta
+    say("decode int4 tiles, sum order", n, h, u, act)
+    g = torch.Generator().manual_seed(n + h + u)
+    e, k = 8, 2
+    idx = torch.stack([torch.randperm(e - 1, generator=g)[:k] for _ in range(n)]).int()
+    up, down = _whole_weights(g, e, h, u, act)
+    x = (torch.randn(n, h, generator=g) * 0.05).to(torch.bfloat16)
+    w = torch.rand(n, k, generator=g) + 0.1
+    got = []
+    for tiles in (False, True):
+        ex, keep = _whole_experts("int4", act, up, down, 64, tiles)
+        got.append(_run_delta(n8, ex, x.to(dev), idx.to(dev), w.to(dev)))
+    assert torch.equal(*got), float((got[0] != got[1]).float().mean())

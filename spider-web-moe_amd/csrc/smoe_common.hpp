@@ -146,10 +146,16 @@ __device__ __forceinline__ float wave_max(float v) {
   v = fmaxf(v, dpp_f<kDppMirror>(v));
   return fmaxf(fmaxf(lane_f(v, 0), lane_f(v, 16)), fmaxf(lane_f(v, 32), lane_f(v, 48)));
 }
-// (value, index) arg-max over the wave; ties -> lowest index.  NaN never wins.
-// Branch-free (bitwise, no short circuit): a branch here becomes exec-mask
-// bookkeeping whose scalar ops wait on each vector compare.
-__device__ __forceinline__ void argmax_take(float& v, int& i, float ov, int oi) {
+// The order of (value, index) pairs in every selection: the larger value
+// first, ties to the lower index; select_key puts NaN at +infinity, so the
+// order is total and lanes that exchange pairs in any sequence end with the
+// same one (argmax_take itself leaves a lane that holds a NaN with its own
+// pair).  One operation per pick: in argmax_take, once per exchange, it cost
+// 1-2% of the decode calls.  Branch-free (bitwise, no short circuit): a branch
+// here becomes exec-mask bookkeeping whose scalar ops wait on each vector
+// compare.  Both are compiled for the host too, where a test runs them.
+__host__ __device__ __forceinline__ float select_key(float v) { return fminf(v, INFINITY); }
+__host__ __device__ __forceinline__ void argmax_take(float& v, int& i, float ov, int oi) {
   const bool take = (ov > v) | ((ov == v) & (oi < i));
   v = take ? ov : v;
   i = take ? oi : i;
@@ -187,6 +193,7 @@ __device__ __forceinline__ float seg_sum(float v) {
 template <int SEG>
 __device__ __forceinline__ void seg_argmax(float& v, int& i) {
   static_assert(SEG == 16 || SEG == 32 || SEG == 64, "segment");
+  v = select_key(v);
   argmax_dpp<kDppXor1>(v, i);
   argmax_dpp<kDppXor2>(v, i);
   argmax_dpp<kDppHalfMirror>(v, i);
@@ -208,10 +215,7 @@ __device__ __forceinline__ void wide_argmax(const float (&x)[V], const bool (&ca
   ci = kWideBig;
 #pragma unroll
   for (int v = 0; v < V; ++v)
-    if (cand[v] && (ci == kWideBig || x[v] > cv)) {
-      cv = x[v];
-      ci = lane + 64 * v;
-    }
+    argmax_take(cv, ci, cand[v] ? select_key(x[v]) : -INFINITY, cand[v] ? lane + 64 * v : kWideBig);
   seg_argmax<64>(cv, ci);
 }
 
@@ -277,19 +281,6 @@ typedef __attribute__((address_space(1))) void* gbl_vptr;
 template <int CPR>
 __device__ __forceinline__ int sw_chunk(int r, int c) {
   return c ^ ((r / (16 / CPR)) & (CPR - 1));
-}
-
-__device__ __forceinline__ void wave_argmax(float& v, int& i) {
-  argmax_dpp<kDppXor1>(v, i);
-  argmax_dpp<kDppXor2>(v, i);
-  argmax_dpp<kDppHalfMirror>(v, i);
-  argmax_dpp<kDppMirror>(v, i);
-  float bv = lane_f(v, 0);
-  int bi = __builtin_amdgcn_readlane(i, 0);
-#pragma unroll
-  for (int r = 16; r < 64; r += 16) argmax_take(bv, bi, lane_f(v, r), __builtin_amdgcn_readlane(i, r));
-  v = bv;
-  i = bi;
 }
 
 // erf by Abramowitz & Stegun, Handbook of Mathematical Functions, eq. 7.1.26:

@@ -306,8 +306,8 @@ __global__ __launch_bounds__(1024) void k_decode_front(const DecFront a) {
         }
     } else {
       const int s = strip - 1;
-      const bool sel_src = (m >> s) & 1ull;
       const int rank = __popcll(m & ((1ull << s) - 1ull));
+      const bool sel_src = ((m >> s) & 1ull) && rank < a.K;
       topm_row<SEG>(lt[1][j][ec], t, ok, sel_src, rank, E, a.K, a.M, a.sel_idx, a.sel_w);
     }
   }

@@ -110,7 +110,7 @@ __global__ __launch_bounds__(256) void k_route_topk_w(const float* __restrict__ 
     wide_ranks<V>(sel, rank);
 #pragma unroll
     for (int v = 0; v < V; ++v)
-      if (sel[v]) {
+      if (sel[v] && rank[v] < K) {
         tok_e[static_cast<int64_t>(t) * K + rank[v]] = lane + 64 * v;
         tok_ew[static_cast<int64_t>(t) * K + rank[v]] = ex[v] / sum / denom;
       }

@@ -61,8 +61,9 @@ __device__ __forceinline__ uint64_t topk_seg(float v, int t, bool ok, bool live,
   const uint64_t segm = SEG == 64 ? ~0ull : ((1ull << SEG) - 1);
   const uint64_t m = (__ballot(sel) >> sbase) & segm;
   if (!tok_e) return m;  // top-k only (the decode front: its plan kernel sorts the sources)
-  if (ok && live && sel) {
-    const int rank = __popcll(m & ((1ull << e) - 1));
+  // K distinct experts; the list's bound does not rest on that alone
+  const int rank = __popcll(m & ((1ull << e) - 1));
+  if (ok && live && sel && rank < K) {
     tok_e[static_cast<int64_t>(t) * K + rank] = e;
     tok_ew[static_cast<int64_t>(t) * K + rank] = p / denom;
     if (tok_e2) {
@@ -132,8 +133,8 @@ __device__ __forceinline__ void topm_seg(const float (&v)[KB], const int (&row)[
   const uint64_t segm = SEG == 64 ? ~0ull : ((1ull << SEG) - 1);
   const uint64_t m = (__ballot(nz) >> sbase) & segm;
   const int cnt = __popcll(m);
-  if (ok && nz) {
-    const int rank = __popcll(m & ((1ull << d) - 1));
+  const int rank = __popcll(m & ((1ull << d) - 1));
+  if (ok && nz && rank < S) {
     tok_d[static_cast<int64_t>(t) * S + rank] = d;
     tok_dc[static_cast<int64_t>(t) * S + rank] = c;
     if (tok_d2) {

@@ -622,6 +622,56 @@ def test_stage_entries_compose_block_forward(spec):
     assert float(row_ratio(delta.float().cpu()[ok], aux.delta[ok]).max()) <= DELTA_TOL
 
 
+# One case per route of the routing: the decode loop (16-, 32- and 64-lane
+# segments), the front without it (H 192), dense logits + chunk routing in
+# bf16 and fp32 (one chunk and several), the one-pass prefill front, the
+# separate stages, and more than 64 experts.
+NAN_CASES = [dict(n=9), dict(n=64, e=32, k=4), dict(n=48, e=64, m=4), dict(n=37, hid=192),
+             dict(n=200), dict(n=777, e=8, k=3), dict(n=130, dtype="f32", act="gelu", e=8, m=3),
+             dict(n=40, dtype="f32", act="gelu", e=16), dict(n=2500), dict(n=300, e=32, k=4),
+             dict(n=100, e=96, k=3)]
+
+
+@pytest.mark.parametrize("case", NAN_CASES, ids=lambda c: "-".join(f"{k}{v}" for k, v in c.items()))
+def test_nan_and_inf_tokens_leave_the_others_alone(case):
+    """Tokens whose hidden states hold a NaN (every logit NaN) or two
+    infinities (a mix of NaN and infinite logits) select K distinct experts
+    like any token: the plans stay whole and every other token keeps the bits
+    it has in a clean batch; their own outputs are NaN."""
+    from spider_moe_amd.workloads import make_block
+    say("nan tokens", case)
+    n, dtype = case["n"], case.get("dtype", "bf16")
+    wl = make_block("c1", tokens=n, hidden_size=case.get("hid", 256), num_experts=case.get("e", 16),
+                    top_k=case.get("k", 2), edges_per_expert=case.get("m", 2), expert_ffn_size=256,
+                    num_loops=3, expert_activation=case.get("act", "swiglu"), dtype=dtype, experts=dtype)
+    layer, h = wl.layer, wl.h.clone()
+    odd = sorted({0, 5, n // 2, n - 1} | {t for t in (62, 63, 64, 127, 128, 191) if t < n})
+    for j, t in enumerate(odd):
+        if j % 2:
+            h[t, 0, 3:5] = float("inf")
+        else:
+            h[t, 0, 7] = float("nan")
+    ok = torch.ones(n, dtype=torch.bool, device=dev)
+    ok[odd] = False
+    with torch.no_grad():
+        clean = layer.forward_loops(wl.h, wl.x0)
+        got = layer.forward_loops(h, wl.x0)
+        one = layer(h, wl.x0, 0)
+    torch.cuda.synchronize()
+    assert bool(clean.isfinite().all()) and torch.equal(got[ok], clean[ok])
+    assert bool(got[~ok].isnan().all()) and bool(one[~ok].isnan().all())
+    r = layer.last_routing()
+    top = r["top_idx"].long().cpu().view(n, -1)
+    assert bool(((top >= 0) & (top < layer.num_experts)).all())
+    srt = top.sort(-1).values
+    assert bool((srt[:, 1:] > srt[:, :-1]).all())  # distinct
+    # the expert plan holds every (token, expert) once, experts ascending
+    off, rows = r["e_off"].cpu().tolist(), r["e_rows"].cpu().tolist()
+    assert off[-1] == n * layer.top_k
+    for x in range(layer.num_experts):
+        assert rows[off[x]:off[x + 1]] == (top == x).any(-1).nonzero().flatten().tolist(), x
+
+
 # ------------------------------------------------ early-exit decode ----
 EXIT_CASES = [dict(kind="bf16", tokens=64), dict(kind="bf16", tokens=300),
               dict(kind="bf16", tokens=48, hid=512, e=32, k=4, m=2),

@@ -2001,14 +2001,16 @@ int stream4_tn(const GemmArgs& a) {
   return cost(3) < cost(4) ? 3 : 4;
 }
 
-// Whether the int4 stream kernel takes the GEMM: every 16-byte (weights and
-// activations) load it issues aligned, K in 64-wide steps, the strip's scales
-// within its LDS table.  Two workgroups per CU (one's dequant and waits
-// overlap the other's MFMAs): LDS per workgroup 3 x 20 KB + 16 KB scales.
+// Whether the int4 stream kernel takes the GEMM: every 16-byte load it issues
+// (weights and activations by DMA, biases) aligned, K in 64-wide steps, the
+// strip's scales within its LDS table.  Codes come 32 to 16 bytes.  Two
+// workgroups per CU (one's dequant and waits overlap the other's MFMAs): LDS
+// per workgroup 3 x 20 KB + 16 KB scales.
 bool stream4_fits(const GemmArgs& a) {
+  const auto odd = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 != 0; };
   if (a.fmt != SMOE_INT4 || a.K % 64 || a.N_out % 4 || a.ldo % 4 || a.lda % 8) return false;
-  if (a.ldw % 16 || a.w_gstride % 16 || a.group_size % 16) return false;
-  if (a.bias && a.bias_gstride % 4) return false;  // 16-byte bias loads
+  if (a.ldw % 32 || a.w_gstride % 32 || a.group_size % 16 || odd(a.A) || odd(a.W)) return false;
+  if (a.bias && (a.bias_gstride % 4 || odd(a.bias))) return false;
   return 256 * (a.K / a.group_size) <= kStreamScaleMax && !(a.group_size & (a.group_size - 1));
 }
 

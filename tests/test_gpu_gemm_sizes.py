@@ -363,3 +363,36 @@ def test_decode_int4_tiles_sum_order(n, h, u, act):
         ex, keep = _whole_experts("int4", act, up, down, 64, tiles)
         got.append(_run_delta(n8, ex, x.to(dev), idx.to(dev), w.to(dev)))
     assert torch.equal(*got), float((got[0] != got[1]).float().mean())
+
+
+# int4 experts whose codes or biases lie off 16-byte boundaries, at the row
+# counts of the int4 stream kernel (16-byte loads): a kernel without them
+@pytest.mark.parametrize("off", ["codes", "bias"])
+def test_int4_stream_unaligned_operands(off):
+    from spider_moe_amd import _native as n8
+    from test_gpu_kernels import _run_delta
+    say("int4 stream, unaligned", off)
+    e, n, h, u = 4, 300, 256, 320
+    g = torch.Generator().manual_seed(3)
+    idx = torch.randint(0, e, (n, 1), generator=g).int()
+    up, down = _whole_weights(g, e, h, u, "gelu")
+    x = (torch.randn(n, h, generator=g) * 0.05).to(torch.bfloat16)
+    w = torch.rand(n, 1, generator=g) + 0.1
+    ex, (mats, kw) = _whole_experts("int4", "gelu", up, down, 64)
+    bu, bd = torch.randn(e, u, generator=g), torch.randn(e, h, generator=g)
+    bias = [torch.nn.functional.pad(b.flatten(), (1, 0)).to(dev)[1:] for b in (bu, bd)]
+    if off == "codes":
+        mats = [torch.nn.functional.pad(m.flatten(), (8, 0))[8:] for m in mats]
+        bias = [b.clone() for b in bias]
+        ex.w_up, ex.w_down = mats[0].data_ptr(), mats[1].data_ptr()
+    ex.b_up, ex.b_down = bias[0].data_ptr(), bias[1].data_ptr()
+    assert ex.w_up % 16 == (8 if off == "codes" else 0) and ex.b_up % 16 == (0 if off == "codes" else 4)
+    y = _run_delta(n8, ex, x.to(dev), idx.to(dev), w.to(dev)).double()
+    for i in range(e):
+        r = (idx[:, 0] == i).nonzero().squeeze(-1)
+        a = torch.nn.functional.gelu(x[r].double() @ up[i].double().t() + bu[i].double())
+        ref = (a @ down[i].double().t() + bd[i].double()) * w[r].double()
+        mag = (a.abs() @ down[i].abs().double().t() + bd[i].abs().double()) * w[r].double()
+        # bf16 activations and rows: 2^-9 of each product and of the result
+        bound = (2.0 ** -9 + (2 * u + 2 * h) * 2.0 ** -24 + 1e-5) * mag + 2.0 ** -9 * ref.abs() + 1e-6
+        assert bool(((y[r] - ref).abs() <= 1.01 * bound).all()), float(((y[r] - ref).abs() / bound).max())

@@ -396,3 +396,28 @@ def test_int4_stream_unaligned_operands(off):
         # bf16 activations and rows: 2^-9 of each product and of the result
         bound = (2.0 ** -9 + (2 * u + 2 * h) * 2.0 ** -24 + 1e-5) * mag + 2.0 ** -9 * ref.abs() + 1e-6
         assert bool(((y[r] - ref).abs() <= 1.01 * bound).all()), float(((y[r] - ref).abs() / bound).max())
+
+
+# 33-128 rows per group, bf16 rows of an odd number of 8-byte pieces: the same
+# bits as with 4 channels more (the down weights pick one channel each, so the
+# delta is the up product's row, scaled)
+@pytest.mark.parametrize("n,h,u", [(160, 320, 324), (500, 128, 1004)])
+def test_grouped_mid_rows_four_channel_stores(n, h, u):
+    from spider_moe_amd import _native as n8
+    from test_gpu_kernels import _experts_struct, _run_delta
+    say("mid rows, 4-channel stores", n, h, u)
+    g = torch.Generator().manual_seed(n + u)
+    e = 4
+    idx = torch.multinomial(torch.tensor([.5, .3, .2, 0.]), n, True, generator=g).int().view(n, 1)
+    x = torch.randn(n, h, generator=g).to(torch.bfloat16)
+    w = torch.rand(n, 1, generator=g) + 0.1
+    up = (torch.randn(e, u + 4, h, generator=g) * h ** -0.5).to(torch.bfloat16)
+    bu = torch.randn(e, u + 4, generator=g)
+    got = []
+    for c in (u, u + 4):
+        down = torch.zeros(e, h, c, dtype=torch.bfloat16)
+        down[:, torch.arange(h), torch.arange(h) + u - h] = 1
+        keep = [t.contiguous().to(dev) for t in (up[:, :c], down, bu[:, :c])]
+        ex = _experts_struct(n8, n8.BF16, n8.ACT_GELU, e, h, c, keep[0], keep[1], b_up=keep[2])
+        got.append(_run_delta(n8, ex, x.to(dev), idx.to(dev), w.to(dev)))
+    assert float(got[0].abs().max()) > 0 and torch.equal(*got), float((got[0] != got[1]).float().mean())

@@ -813,14 +813,14 @@ int launch_plan(const int32_t* tok_g, const float* tok_w, int N, int S, int G, i
   if (G < 1 || G > kPlanMaxG || S < 1 || S > kPlanMaxS || N < 0) return SMOE_EINVAL;
   const int C = (N + 63) / 64;
   // One wave for a single chunk over <= 64 groups; one workgroup while its
-  // rank work (C x G ballots) stays small; the three-kernel form spreads
-  // larger plans over the chip.
+  // rank work (C x G ballots) stays small and its scan holds every chunk (one
+  // per lane); the three-kernel form spreads larger plans over the chip.
   if (N <= 64 && G <= 64) {
     hipLaunchKernelGGL(k_plan64, dim3(1), dim3(64), 0, s, tok_g, tok_w, N, S, G, drop, cnt, acnt,
                        off, rows, roww, tokrow);
     return hipGetLastError() == hipSuccess ? SMOE_OK : SMOE_EHIP;
   }
-  if (C * G <= 512) {
+  if (C <= 64 && C * G <= 512) {
     const int win = plan_small_win(C, G);
     hipLaunchKernelGGL(k_plan_small, dim3(1), dim3(1024), 0, s, tok_g, tok_w, N, S, G, drop, win,
                        cnt, acnt, off, rows, roww, tokrow);

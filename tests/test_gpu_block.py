@@ -522,6 +522,23 @@ def test_block_wide_experts(e, k, m, dtype, act):
         assert int((rep.get("experts_touched", 1))) >= 1
 
 
+@pytest.mark.parametrize("n,e,k,m,dtype", [(4096, 4, 2, 2, "f32"), (4097, 4, 1, 2, "bf16"),
+                                           (8000, 4, 2, 2, "f32"), (5000, 7, 2, 3, "bf16"),
+                                           (4160, 1, 1, 1, "bf16"), (16000, 2, 1, 1, "bf16")])
+def test_block_many_chunks_over_few_experts(n, e, k, m, dtype):
+    """More than 64 token chunks over at most 7 experts: the plans' rank work
+    is small (C * E <= 512) but a one-workgroup scan (a chunk per lane) does
+    not hold them."""
+    from spider_moe_amd.workloads import make_block
+    say("many chunks", n, e, k, m, dtype)
+    wl = make_block("c1", tokens=n, hidden_size=64, num_experts=e, top_k=k, edges_per_expert=m,
+                    expert_ffn_size=64, num_loops=1, expert_activation="gelu", experts=dtype, dtype=dtype)
+    _check_loop(wl.layer, wl.h, wl.x0, 0, 1e-4 if dtype == "f32" else 1e-2)
+    rt = wl.layer.last_routing()
+    assert int(rt["e_cnt"].sum()) == n * k
+    assert int(rt["d_cnt"].sum()) == int((rt["tok_d"] >= 0).sum())
+
+
 def test_block_rejects_unsupported_shapes_clearly():
     """Shapes past the kernels' limits raise a ValueError that names them,
     before any launch."""

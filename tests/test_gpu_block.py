@@ -791,6 +791,55 @@ def test_exit_gate_partial_teacher_forced(case):
         "bit-identical rows", int((g[ok] == pick[ok]).all(-1).sum()), "of", int(ok.sum()))
 
 
+@pytest.mark.parametrize("dtype,n,e,k,m", [("bf16", 65, 16, 2, 2), ("bf16", 300, 16, 2, 2),
+                                           ("bf16", 777, 8, 3, 3), ("bf16", 2048, 16, 2, 2),
+                                           ("f32", 5, 8, 2, 3), ("f32", 64, 8, 2, 3), ("f32", 333, 16, 2, 4)])
+def test_exit_gate_dense_front(dtype, n, e, k, m):
+    """The exit gate over the dense logits + chunk routing launches: every
+    token of the second 64-token chunk (n > 64) leaves after the first loop, a
+    third of the others after each.  A token's output is bit for bit the state
+    it has after its last loop in the ungated run, which the decisions follow
+    (test_exit_gate_partial_teacher_forced's rule; fp32: no rounded logit)."""
+    from spider_moe_amd import _native as nat
+    from spider_moe_amd.workloads import make_block
+    say("exit, dense front", dtype, n, e, k, m)
+    f32, thr, hid = dtype == "f32", 0.6, 256
+    wl = make_block("c1", tokens=n, hidden_size=hid, num_experts=e, top_k=k, edges_per_expert=m,
+                    expert_ffn_size=256, num_loops=3, expert_activation="gelu" if f32 else "swiglu",
+                    experts=dtype, dtype=dtype)
+    layer, h, x0, r = wl.layer, wl.h.clone(), wl.x0, 3
+    h[64:128, 0, 0] = 50.0
+    ew = torch.randn(hid, generator=torch.Generator().manual_seed(9)) / hid ** 0.5
+    ew[0] = 4.0
+    _set_exit(layer, ew, 0.0)
+    ew_stored = layer.exit_head.weight.detach().float().cpu().reshape(-1)
+    timer = nat.StageTimer(stages=["router_gemm", "edge_logits", "front_gemm", "front_route"], capacity=64)
+    timer.start()
+    with torch.no_grad():
+        out, active, loops = layer.forward_loops_exit(h, x0, thr)
+    assert set(timer.stop()) == {"front_gemm", "front_route"}
+    states, cur = [], h
+    with torch.no_grad():
+        for li in range(r):
+            cur = layer(cur, x0, li)
+            states.append(cur.reshape(-1, hid).float().cpu())
+    torch.cuda.synchronize()
+    z_thr = float(np.log(thr / (1 - thr)))
+    # bf16: two ulps of the rounded logit; fp32: the logit's own sums
+    band = 2.0 * 2.0 ** (np.floor(np.log2(abs(z_thr))) - 7) if not f32 else 1e-4
+    exp, tie, done = torch.full((n,), r), torch.zeros(n).bool(), torch.zeros(n).bool()
+    for li in range(r):
+        tie |= ~done & ((B.exit_logit(states[li], ew_stored, 0.0) - z_thr).abs() < band)
+        ex = ~done & (torch.sigmoid(B.exit_logit(states[li], ew_stored, 0.0, bf16=not f32)) > thr)
+        exp[ex] = li + 1
+        done |= ex
+    loops, ok = loops.cpu().long(), ~tie
+    assert torch.equal(loops[ok], exp[ok]) and torch.equal(active.cpu()[ok] != 0, ~done[ok])
+    assert bool((loops[64:128] == 1).all()) and (n < 64 or set(loops.tolist()) == {1, 2, 3})
+    pick = torch.stack([states[int(l) - 1][t] for t, l in enumerate(loops.tolist())])
+    assert torch.equal(out.reshape(-1, hid).float().cpu(), pick)
+
+
 def test_decode_graph_replays_match_eager():
     """The R-loop decode with the exit gate captured as one HIP graph
     (spider_infer/cuda_graph.py:79-130): replays with new inputs, with eager

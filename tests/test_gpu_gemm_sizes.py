@@ -68,11 +68,14 @@ def test_f32_grouped_tile_edges(n, h, u, e, k):
 
 # 33-255 rows per group on average, and any row count of fp8 / int4 without
 # tile copies: groups of 0, 1, 64, 65, .. rows (tiles of 64 and 128 rows), K
-# of one to five 64-k stages and channels off the 128-wide strips; 139 rows
+# of one to five 64-k stages and channels off the 128-wide strips; 140 rows
 # per group on average: (192, 320) makes fewer 64 x 128 tiles than CUs (64 x
 # 64 tiles), (128, 2696) more (3 stages), (64, 5312) more than two per CU (2
 # stages), (128, 456) a partial strip; a third of the rows, (128, 2696): the
-# 64-row SwiGLU tiles
+# 64-row SwiGLU tiles.  int4 has 64-k scale groups here: the down products of
+# U 2752 and 5312 (43 and 83 along K) run on the general kernel, and a third
+# of the rows on the int4 stream kernel (test_grouped_mid_int4_scales has the
+# scale table's sizes)
 @pytest.mark.parametrize("h,u,part", [(192, 320, 1), (128, 2696, 1), (64, 5312, 1), (128, 456, 1),
                                       (128, 2696, 3)])
 @pytest.mark.parametrize("fmt,act", [("bf16", "gelu"), ("bf16", "swiglu"), ("fp8", "gelu"),
@@ -393,9 +396,10 @@ def test_int4_stream_unaligned_operands(off):
         a = torch.nn.functional.gelu(x[r].double() @ up[i].double().t() + bu[i].double())
         ref = (a @ down[i].double().t() + bd[i].double()) * w[r].double()
         mag = (a.abs() @ down[i].abs().double().t() + bd[i].abs().double()) * w[r].double()
-        # bf16 activations and rows: 2^-9 of each product and of the result
-        bound = (2.0 ** -9 + (2 * u + 2 * h) * 2.0 ** -24 + 1e-5) * mag + 2.0 ** -9 * ref.abs() + 1e-6
-        assert bool(((y[r] - ref).abs() <= 1.01 * bound).all()), float(((y[r] - ref).abs() / bound).max())
+        # bf16 (8 significant bits: 2^-8) activations, of each product, and rows;
+        # f32 sums of u and h terms and the f32 activation: far below
+        bound = (2.0 ** -8 + (2 * u + 2 * h) * 2.0 ** -24 + 1e-5) * mag + 2.0 ** -8 * ref.abs() + 1e-6
+        assert bool(((y[r] - ref).abs() <= bound).all()), float(((y[r] - ref).abs() / bound).max())
 
 
 # 33-128 rows per group, bf16 rows of an odd number of 8-byte pieces: the same
@@ -421,3 +425,49 @@ def test_grouped_mid_rows_four_channel_stores(n, h, u):
         ex = _experts_struct(n8, n8.BF16, n8.ACT_GELU, e, h, c, keep[0], keep[1], b_up=keep[2])
         got.append(_run_delta(n8, ex, x.to(dev), idx.to(dev), w.to(dev)))
     assert float(got[0].abs().max()) > 0 and torch.equal(*got), float((got[0] != got[1]).float().mean())
+
+
+# int4 at 140 rows per group without tile copies: scale tables of one to 32
+# groups along the down product's K, the most that the tiles hold (64 x 32, 128 x
+# 22), and 33 (the general kernel), scales of both types
+@pytest.mark.parametrize("u,group", [(128, 128), (192, 64), (2048, 64), (2816, 128), (4096, 128), (2112, 64)])
+@pytest.mark.parametrize("sdt", [torch.float16, torch.float32])
+def test_grouped_mid_int4_scales(u, group, sdt):
+    from spider_moe_amd import _native as n8
+    from spider_moe_amd.quant import quantize_int4
+    from test_gpu_kernels import _experts_struct, _run_delta
+    say("int4 mid scales", u, group, sdt)
+    g = torch.Generator().manual_seed(u + group)
+    h, rows = 128, [300, 130, 0, 260, 65, 300, 1, 64]
+    e, n = len(rows), sum(rows)
+    idx = torch.cat([torch.full((r,), x, dtype=torch.int32) for x, r in enumerate(rows)])
+    idx = idx[torch.randperm(n, generator=g)].view(n, 1)
+    x, w = torch.randn(n, h, generator=g).to(torch.bfloat16), torch.rand(n, 1, generator=g) + 0.1
+    bu, bd = torch.randn(e, u, generator=g) * 0.1, torch.randn(e, h, generator=g) * 0.1
+    vals, packed, scales = [], [], []
+    for o, k in ((u, h), (h, u)):
+        # magnitudes that differ from one scale group to the next
+        m = torch.randn(e, o, k, generator=g) * k ** -0.5 * (torch.rand(e, o, k // group, 1, generator=g) * 4 + 0.1) \
+            .expand(-1, -1, -1, group).reshape(e, o, k)
+        q = quantize_int4(m, group, sdt)
+        b = q.packed.view(torch.uint8).int()
+        nib = torch.stack([b & 15, b >> 4], -1).view(m.shape)
+        nib = torch.where(nib > 7, nib - 16, nib).float()
+        vals.append((nib * q.scales.float().repeat_interleave(group, -1)).to(torch.bfloat16).double())
+        packed.append(q.packed.contiguous().to(dev))
+        scales.append(q.scales.contiguous().to(dev))
+    bias = [bu.to(dev), bd.to(dev)]
+    ex = _experts_struct(n8, n8.INT4, n8.ACT_GELU, e, h, u, *packed, s_up=scales[0], s_down=scales[1],
+                         b_up=bias[0], b_down=bias[1], group=group,
+                         scale_dtype=n8.F16 if sdt == torch.float16 else n8.F32)
+    y = _run_delta(n8, ex, x.to(dev), idx.to(dev), w.to(dev)).double()
+    for i in range(e):
+        r = (idx[:, 0] == i).nonzero().squeeze(-1)
+        if not len(r):
+            continue
+        a = torch.nn.functional.gelu(x[r].double() @ vals[0][i].t() + bu[i].double())
+        ref = (a @ vals[1][i].t() + bd[i].double()) * w[r].double()
+        mag = (a.abs() @ vals[1][i].abs().t() + bd[i].abs().double()) * w[r].double()
+        # as in test_int4_stream_unaligned_operands
+        bound = (2.0 ** -8 + (2 * u + 2 * h) * 2.0 ** -24 + 1e-5) * mag + 2.0 ** -8 * ref.abs() + 1e-6
+        assert bool(((y[r] - ref).abs() <= bound).all()), (i, float(((y[r] - ref).abs() / bound).max()))

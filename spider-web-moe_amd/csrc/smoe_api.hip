@@ -226,6 +226,8 @@ bool prefill_front_ok(const smoe_block* b, int N) {
 // took six launches, 52 us of a bf16 loop at 777 tokens and 61 us of an fp32
 // one at 2048 (E 8), against 25 and 21 us for the three; past it the
 // prefill front reads h once instead of once per 16 channels.
+// Past 256 selected rows per expert the logits' last place is not that of the
+// separate stages (launch_front_dense).
 // The logits wait in the proj region and the second plan's counts in act
 // (both written later in the loop), so the workspace is no larger.
 bool dense_front_ok(const smoe_block* b, int N) {

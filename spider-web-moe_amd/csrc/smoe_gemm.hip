@@ -1554,11 +1554,11 @@ __global__ __launch_bounds__(256, 2) void k_gemm_stream4(const GemmArgs p) {
 }
 
 // ------------------------------------------------- fp32 / any shape ----
-// SIMT tile GEMM with fp32 FMAs: the fp32 models' path (FMT = SMOE_F32, A
-// and W fp32) and the fallback for bf16 shapes the MFMA kernels do not take
-// (K or a row pitch not a multiple of their vector width; FMT = SMOE_BF16,
-// A and W bf16).  Any K and N_out: k past K reads as 0, which leaves every
-// sum unchanged (fma(a, 0, acc) == acc).
+// SIMT tile GEMM with fp32 FMAs: the fallback for fp32 shapes off the matrix
+// tiles' grid (smoe_gemm_f32.hip; FMT = SMOE_F32, A and W fp32) and for bf16
+// shapes the MFMA kernels do not take (K or a row pitch not a multiple of
+// their vector width; FMT = SMOE_BF16, A and W bf16).  Any K and N_out: k past
+// K reads as 0, which leaves every sum unchanged (fma(a, 0, acc) == acc).
 template <int FMT>
 __device__ __forceinline__ float elem(const void* base, int64_t i) {
   if constexpr (FMT == SMOE_F32) return reinterpret_cast<const float*>(base)[i];
@@ -2054,7 +2054,9 @@ int launch_front_dense(const GemmArgs& a, hipStream_t s) {
   if (a.fmt == SMOE_F32) return launch_gemm_f32_front(a, s);
   if (a.fmt != SMOE_BF16 || a.K % 64 || a.lda % 8 || a.ldw % 8 || a.ldw2 % 8) return SMOE_EINVAL;
   // the front GEMM's tiles: every output is summed as the separate stages'
-  // skinny GEMMs sum it, so the logits keep their bits
+  // skinny GEMMs sum it, so the logits have their bits while those stages run
+  // on skinny tiles (up to 256 selected rows per expert and 4095 tokens; past
+  // either they differ in the order of the f32 sums)
   return launch_skinny_fmt<SMOE_BF16, 1, 1, 4, 4>(a, s);
 }
 

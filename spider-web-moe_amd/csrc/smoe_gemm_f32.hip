@@ -35,9 +35,10 @@ __device__ __forceinline__ bool vec_out(const GemmArgs& p) {
 // BM x BN tile, 4 waves in a 2 x 2 grid, K in 32-wide stages (128-byte rows)
 // that go global -> LDS by DMA through a 3-stage ring, two stages in flight
 // while one computes.  Bound: the fp32 matrix pipe (256 flop per clock and
-// CU); a 64 x 64 tile reads 4 KB of fragments per 16-k block for 128 MFMAs
-// (1024 pipe cycles a SIMD), so neither LDS nor L2 is near its limit, and 48 KB of
-// LDS let three workgroups share a CU and hide each other's waits.  Against
+// CU); a wave of a 64 x 64 tile reads 4 KB of fragments per 16-k block for 16
+// MFMAs (512 cycles of its SIMD's pipe), the workgroup 16 KB in that time, a
+// quarter of what LDS delivers, and 48 KB of LDS let three workgroups share a
+// CU and hide each other's waits.  Against
 // the VALU tile kernel (scalar loads, one barrier pair per 16 k): H 256, U
 // 512, E 8, 2048 tokens (about 512 rows per expert, 1200 per destination),
 // us per launch: up 63 -> 21.5, down 98.5 -> 22.9, edge projection 61.7 ->

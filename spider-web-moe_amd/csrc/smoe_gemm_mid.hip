@@ -1,7 +1,8 @@
 // Grouped GEMMs between the weight streams of decode steps and the large
 // prefill tiles: a few dozen to a few hundred rows per group, where neither
 // the weights nor the matrix pipe alone sets the time, and the fp8 / int4
-// GEMMs of any row count that have no tile copy.
+// GEMMs of any row count that have no tile copy (int4: with at most
+// kMidScaleMax scale groups along K).
 #include "smoe_common.hpp"
 #include "smoe_gemm.hpp"
 #include "smoe_internal.hpp"
@@ -16,7 +17,11 @@ template <int FMT>
 constexpr int mid_wb() {  // bytes of one channel's 64-k slice
   return FMT == SMOE_BF16 ? 128 : (FMT == SMOE_FP8_E4M3 ? 64 : 32);
 }
-constexpr int kMidScaleMax = 32;  // int4 scale groups along K
+// int4 scale groups along K: the [groups, 128] table of a tile is 16 KB of LDS
+// beside the ring (three workgroups of 2 stages per CU).  Wider tables, e.g. the
+// 44 groups of U 2816 in groups of 64, leave that GEMM on the general kernel:
+// 777 tokens, H 1024, 16 int4 experts 1224 us in groups of 64, 774 in groups of 128.
+constexpr int kMidScaleMax = 32;
 
 // The tile of workgroup bid: tiles go group by group, within a group strip by
 // strip and the strip's row tiles next to each other, so that a weight strip
